@@ -830,18 +830,18 @@ void conv1d_mfma_persist_kernel(ConvLaunch a, int n_tx, int n_ty, int stage_floa
 // Mean and 1 / den of a LayerNorm over C channels for column i0 + tid % BN,
 // from the float64 (sum, sum of squares) of ntile 32-row tiles, double2
 // [B][ntile][L] (ConvLaunch::stat_out).  NP = NT / BN threads per column:
-// thread (p, col) adds tiles p, p + NP, ... with all its loads in flight,
-// then one thread adds the NP partials in p order -- a fixed grouping, so
+// thread (p, col) adds tiles p, p + NP, ... four loads in flight at a time
+// (768 channels are 24 tiles: one pass of the loop in every kernel here), then
+// one thread adds the NP partials in p order -- a fixed grouping, so
 // the result depends on the statistics only.  mean = S / C, var = (Q - S *
 // mean) / C, den = sqrt(var + eps) (the LayerNorm kernels' formulas with the
 // two passes folded into the sums).  scratch: NT double2 + 2 BN floats of
 // LDS; two barriers, every thread of the workgroup calls it.  Columns past L
 // get 0, 0.
-template <int NT, int BN, int kMaxPer = 4>
+template <int NT, int BN>
 __device__ __forceinline__ void ln_column_stats(const double* stat, int ntile, int C, int L, float eps, int b, int i0,
                                                 float* scratch, float& mu, float& rd) {
-  constexpr int NP = NT / BN;
-  // tiles per thread: ntile <= NP * kMaxPer (checked by the launcher)
+  constexpr int NP = NT / BN, kPass = 4;
   const int tid = threadIdx.x;
   const int col = tid % BN, p = tid / BN;
   const int i = i0 + col;
@@ -849,17 +849,19 @@ __device__ __forceinline__ void ln_column_stats(const double* stat, int ntile, i
   double2* part = reinterpret_cast<double2*>(scratch);
   float* out = reinterpret_cast<float*>(part + NT);
   const double2* st = reinterpret_cast<const double2*>(stat) + (long long)b * ntile * L + i;
-  double2 v[kMaxPer];
-#pragma unroll
-  for (int u = 0; u < kMaxPer; ++u) {
-    const int t = p + NP * u;
-    v[u] = icol && t < ntile ? st[(long long)t * L] : make_double2(0.0, 0.0);
-  }
   double S = 0.0, Q = 0.0;
+  for (int t0 = 0; t0 < ntile; t0 += NP * kPass) {
+    double2 v[kPass];
 #pragma unroll
-  for (int u = 0; u < kMaxPer; ++u) {
-    S += v[u].x;
-    Q += v[u].y;
+    for (int u = 0; u < kPass; ++u) {
+      const int t = t0 + p + NP * u;
+      v[u] = icol && t < ntile ? st[(long long)t * L] : make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int u = 0; u < kPass; ++u) {
+      S += v[u].x;
+      Q += v[u].y;
+    }
   }
   part[tid] = make_double2(S, Q);
   __syncthreads();
@@ -2077,8 +2079,7 @@ bool conv1x1_split_ok(const ConvLaunch& a) {
   const ConvGroup& G = a.g[0];
   return a.n_groups == 1 && G.wsp && G.wsc && G.K == 1 && G.in_step <= 1 && G.in_off == 0 && G.out_step == 1 &&
          G.out_off == 0 && G.n_out <= a.L_in && a.C_in > 256 && a.C_in % 64 == 0 && a.C_out % 64 == 0 &&
-         a.in_act == ACT_NONE && a.post == POST_NONE && !a.ln_g && a.B <= 65535 && small_offsets_ok(a) &&
-         (!a.ln_stat || a.ln_ntile <= 64) && (!a.res_stat || a.C_out <= 2048);
+         a.in_act == ACT_NONE && a.post == POST_NONE && !a.ln_g && a.B <= 65535 && small_offsets_ok(a);
 }
 
 bool conv1d_mfma_small_path(const ConvLaunch& a) {

@@ -51,3 +51,24 @@ def test_scale_of_the_values(weights, hub, exponent):
     other.encode(x)
     assert rel_l2(other.read("proj", (1, 768, L)) / s, hub.read("proj", (1, 768, L))) < 1e-6
     other.close()
+
+
+def _other_width(hidden, ffn, L):
+    """rel L2 of a two-layer model of another width against the oracle."""
+    sd = syn.make_hubert_weights(syn.HubertGeometry(conv_dim=64, hidden=hidden, n_layers=2, ffn=ffn), seed=hidden)
+    x = syn.make_hubert_input(400 + 320 * (L - 1), seed=L)
+    with nn_ref.conv_formulation("taps"):
+        want = hubert_ref.HubertRef(sd).encode(x)
+    m = HipHubert(sd)
+    got = m.encode(x)
+    m.close()
+    assert got.shape == want.shape == (1, L, hidden)
+    return rel_l2(got, want)
+
+
+@pytest.mark.parametrize("hidden,ffn,L", [(1152, 4608, 129), (1536, 6144, 129)])
+def test_more_than_1024_channels(hidden, ffn, L):
+    """36 and 48 tiles of LayerNorm statistics, at a frame count at which q/k/v
+    and the FFN run on 64-row tiles of four waves."""
+    # sums of up to 6144 products, as above
+    assert _other_width(hidden, ffn, L) < 5e-6
