@@ -1356,8 +1356,8 @@ __global__ __launch_bounds__(64 * NW) void conv_small_kernel(ConvLaunch a) {
 // 3072, 50 .. a few thousand frames) on split products (conv_split.hip).
 //
 // A workgroup forms 32 TM rows x 32 columns; its NW waves each take a run of
-// 16-channel steps and all of the tile, and the partial tiles are added in wave
-// order in small_conv_epilogue.  Nothing is staged: a lane of the column
+// pairs of 16-channel steps (C_in is a multiple of 64) and all of the tile, and
+// the partial tiles are added in wave order in small_conv_epilogue.  Nothing is staged: a lane of the column
 // operand holds 8 channels of one column, eight loads that are 128 consecutive
 // bytes over its 32 lanes, split in registers; the row operand is one load per
 // part from the packed weights.  So a wave runs its steps without a barrier,
@@ -1384,7 +1384,7 @@ void conv1x1_split_kernel(ConvLaunch a, int n_row, int n_col) {
   const int half = lane >> 5, l32 = lane & 31;
   const int col = i0 + l32;
   const int C_in = a.C_in, n = C_in / 16, nrb = a.C_out / 32;
-  const int s_lo = n * wave / NW, s_hi = n * (wave + 1) / NW;
+  const int s_lo = 2 * (n / 2 * wave / NW), s_hi = 2 * (n / 2 * (wave + 1) / NW);
 
   const float* xb = G.x + (long long)b * a.xb;
   const __amdgpu_buffer_rsrc_t xrs = uniform_rsrc(xb, 4u * (unsigned)((C_in - 1) * (int)a.xc + a.L_in));
@@ -1396,10 +1396,9 @@ void conv1x1_split_kernel(ConvLaunch a, int n_row, int n_col) {
   auto load = [&](int s, int p) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int st = __builtin_amdgcn_readfirstlane(min(s + u, n - 1));
-      const bool on = s + u < s_hi;
+      const int st = __builtin_amdgcn_readfirstlane(s + u);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) xv[p][u][j] = buf_load4(xrs, on ? xo : kBufOut, 4u * (unsigned)((16 * st + j) * (int)a.xc));
+      for (int j = 0; j < 8; ++j) xv[p][u][j] = buf_load4(xrs, xo, 4u * (unsigned)((16 * st + j) * (int)a.xc));
 #pragma unroll
       for (int q = 0; q < 2; ++q)
 #pragma unroll

@@ -72,3 +72,11 @@ def test_more_than_1024_channels(hidden, ffn, L):
     and the FFN run on 64-row tiles of four waves."""
     # sums of up to 6144 products, as above
     assert _other_width(hidden, ffn, L) < 5e-6
+
+
+@pytest.mark.parametrize("hidden,ffn,L", [(384, 1536, 33), (384, 1536, 460), (576, 2304, 40), (576, 2304, 300),
+                                          (960, 3840, 40), (960, 3840, 170), (1344, 5376, 97)])
+def test_uneven_shares_of_the_waves(hidden, ffn, L):
+    """Widths whose 16-channel steps do not divide evenly among the four or
+    eight waves of a tile, with the LayerNorm applied on the way in."""
+    assert _other_width(hidden, ffn, L) < 5e-6
