@@ -123,6 +123,7 @@ void Engine::free_block(void* p, size_t block) {
 }
 
 void Engine::upload(void* dst, const void* src, size_t n) {
+  RVC_CHECK(src, "upload: null source");
   if (n > kStageMax) {
     RVC_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, stream));
     sync();
@@ -137,6 +138,7 @@ void Engine::upload(void* dst, const void* src, size_t n) {
 }
 
 void Engine::download(void* dst, const void* src, size_t n) {
+  RVC_CHECK(dst, "download: null destination");
   if (n > kStageMax) {
     RVC_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, stream));
     sync();
