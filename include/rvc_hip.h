@@ -175,9 +175,10 @@ int32_t rvc_last_error(char* buf, int64_t buf_size);
  * count since creation or the last reset; zeros otherwise */
 int32_t rvc_ts_stats(int64_t h, int64_t* busy_ns_out, int64_t* submits_out);
 int32_t rvc_ts_reset(int64_t h);
-/* replaces rvc_mem_stats (engine/src/ffi.zig:1147): every buffer is its own device allocation, so the
- * suballocator / free-list / staging outputs are 0; buf_count, buf_bytes, max_buf_bytes are the live
- * buffers', direct_bytes adds the engine's weight-packing scratch */
+/* replaces rvc_mem_stats (engine/src/ffi.zig:1147): every buffer is its own device block, so the
+ * suballocator outputs are 0; buf_count, buf_bytes, max_buf_bytes are the live buffers', direct_bytes the
+ * device memory behind them, the freed blocks kept for reuse and the engine's weight-packing scratch;
+ * staging_up and staging_dn the pinned block that serves small transfers both ways */
 int32_t rvc_mem_stats(int64_t h, int64_t* sub_total_out, int64_t* sub_chunks_out, int64_t* sub_free_bytes_out,
                       int64_t* sub_free_blocks_out, int64_t* buf_count_out, int64_t* buf_bytes_out,
                       int64_t* staging_up_out, int64_t* staging_dn_out, int64_t* direct_bytes_out,

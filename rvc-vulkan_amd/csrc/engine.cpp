@@ -87,39 +87,53 @@ size_t Engine::block_size(size_t n) {
   return std::max<size_t>((n + step - 1) / step, 1) * step;
 }
 
+void Engine::drop_oldest() {
+  const PoolBlock b = pool.front();
+  pool_of[b.bytes].pop_front();
+  pool.pop_front();
+  pool_bytes -= b.bytes;
+  (void)hipFree(b.ptr);
+}
+
 void Engine::trim_pool() {
-  for (auto& kv : pool)
-    for (void* p : kv.second) (void)hipFree(p);
-  pool.clear();
-  pool_bytes = 0;
+  while (!pool.empty()) drop_oldest();
+}
+
+void* Engine::dev_malloc(size_t bytes) {
+  void* p = nullptr;
+  hipError_t er = hipMalloc(&p, bytes);
+  if (er != hipSuccess && !pool.empty()) {
+    (void)hipGetLastError();
+    trim_pool();
+    er = hipMalloc(&p, bytes);
+  }
+  if (er != hipSuccess) {
+    (void)hipGetLastError();
+    throw Error(std::string("hipMalloc of ") + std::to_string(bytes) + " bytes: " + hipGetErrorString(er));
+  }
+  return p;
 }
 
 void* Engine::alloc_block(size_t block) {
-  auto it = pool.find(block);
-  if (it != pool.end() && !it->second.empty()) {
-    void* p = it->second.back();
-    it->second.pop_back();
-    pool_bytes -= block;
-    return p;
-  }
-  void* p = nullptr;
-  hipError_t er = hipMalloc(&p, block);
-  if (er != hipSuccess && pool_bytes > 0) {
-    (void)hipGetLastError();
-    trim_pool();
-    er = hipMalloc(&p, block);
-  }
-  if (er != hipSuccess) throw Error(std::string("hipMalloc: ") + hipGetErrorString(er));
+  auto& of = pool_of[block > kPoolBlock ? 0 : block];  // 0: no block is
+  if (of.empty()) return dev_malloc(block);
+  const auto it = of.back();
+  of.pop_back();
+  void* p = it->ptr;
+  pool.erase(it);
+  pool_bytes -= block;
   return p;
 }
 
 void Engine::free_block(void* p, size_t block) {
-  if (block > kPoolBlock || pool_bytes + block > kPoolBytes) {
+  if (block > kPoolBlock) {
     RVC_HIP(hipFree(p));
     return;
   }
-  pool[block].push_back(p);
+  pool.push_back({p, block});
+  pool_of[block].push_back(std::prev(pool.end()));
   pool_bytes += block;
+  while (pool_bytes > kPoolBytes) drop_oldest();
 }
 
 void Engine::upload(void* dst, const void* src, size_t n) {
@@ -172,7 +186,7 @@ void* Engine::scratch_for(size_t bytes) {
     if (scratch) RVC_HIP(hipFree(scratch));
     scratch = nullptr;
     scratch_bytes = 0;
-    RVC_HIP(hipMalloc(&scratch, bytes));
+    scratch = dev_malloc(bytes);
     scratch_bytes = bytes;
   }
   return scratch;
@@ -753,9 +767,7 @@ void op_gru(Engine& e, bool dry, long long a_, long long b_, long long c_, long 
   g.o_d = hdim; g.o_t = 2 * hdim; g.o_j = 1;
   g.T = (int)t; g.H = (int)hdim; g.spin_limit = 1LL << 22;
   if (!e.gru_state) {
-    void* p = nullptr;
-    RVC_HIP(hipMalloc(&p, sizeof(unsigned long long) * (2 * 2 * 256 + 2)));
-    e.gru_state = static_cast<unsigned long long*>(p);
+    e.gru_state = static_cast<unsigned long long*>(e.dev_malloc(sizeof(unsigned long long) * (2 * 2 * 256 + 2)));
   }
   g.state = e.gru_state;
   g.sync = reinterpret_cast<unsigned*>(e.gru_state + 2 * 2 * 256);
@@ -1314,19 +1326,18 @@ int32_t rvc_mem_stats(int64_t h, int64_t* sub_total, int64_t* sub_chunks, int64_
     int64_t* outs[] = {sub_total,  sub_chunks, sub_free_bytes, sub_free_blocks, buf_count,  buf_bytes,
                        staging_up, staging_dn, direct_bytes,   max_buf_bytes,   max_buf_sub};
     for (int64_t* p : outs) RVC_CHECK(p != nullptr, "mem_stats: null output");
-    long long total = 0, mx = 0;
+    long long total = 0, blocks = 0, mx = 0;
     for (auto& kv : e.bufs) {
       total += (long long)kv.second.bytes;
+      blocks += (long long)kv.second.block;
       mx = std::max(mx, (long long)kv.second.bytes);
     }
-    // every buffer is its own device block: no suballocator chunks (the freed
-    // blocks kept for reuse are not a suballocator's, nor is the small pinned
-    // staging a buffer of the caller's)
+    // every buffer is its own device block: no suballocator
     *sub_total = *sub_chunks = *sub_free_bytes = *sub_free_blocks = 0;
     *buf_count = (int64_t)e.bufs.size();
     *buf_bytes = total;
-    *staging_up = *staging_dn = 0;
-    *direct_bytes = total + (long long)e.scratch_bytes;
+    *staging_up = *staging_dn = e.stage ? (int64_t)Engine::kStageBytes : 0;  // one block serves both ways
+    *direct_bytes = blocks + (long long)(e.pool_bytes + e.scratch_bytes);
     *max_buf_bytes = mx;
     *max_buf_sub = 0;
   });

@@ -3,6 +3,8 @@
 // the pending batch of the record/commit API.
 #pragma once
 
+#include <deque>
+#include <list>
 #include <memory>
 #include <unordered_map>
 
@@ -34,10 +36,16 @@ struct Engine {
   // hipFree, in a call of its own; a LayerNorm of [100][192] 50 -> 40 us).  A
   // block goes back to the pool after the stream has been waited for, as it went
   // to hipFree before.
-  // At most kPoolBytes are kept, blocks above kPoolBlock not at all; the pool
-  // is emptied when an allocation fails and with the engine.
+  // At most kPoolBytes are kept, the oldest given back first, blocks above
+  // kPoolBlock not at all; the pool is emptied where any device allocation of
+  // the engine or its sessions fails (dev_malloc), and with the engine.
   static constexpr size_t kPoolBytes = 128u << 20, kPoolBlock = 32u << 20;
-  std::map<size_t, std::vector<void*>> pool;
+  struct PoolBlock {
+    void* ptr;
+    size_t bytes;
+  };
+  std::list<PoolBlock> pool;  // oldest first
+  std::unordered_map<size_t, std::deque<std::list<PoolBlock>::iterator>> pool_of;  // by size, oldest first
   size_t pool_bytes = 0;
   // Pinned staging of small transfers: an upload is copied here and on to the
   // device, by a kernel of the stream and without waiting; a download comes back
@@ -74,8 +82,10 @@ struct Engine {
   // the block size a buffer of n bytes takes: eight steps per power of two (n
   // itself where it is not pooled)
   static size_t block_size(size_t n);
+  void* dev_malloc(size_t bytes);  // hipMalloc, again with the pool emptied where it fails
   void* alloc_block(size_t block);
   void free_block(void* p, size_t block);  // the stream has been waited for
+  void drop_oldest();
   void trim_pool();
   void upload(void* dst, const void* src, size_t n);    // may return before the copy has run
   void download(void* dst, const void* src, size_t n);  // waits for the stream

@@ -60,8 +60,7 @@ struct Vc : SessionBase {
   }
 
   float* dalloc(size_t n) {
-    void* p = nullptr;
-    RVC_HIP(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(float)));
+    void* p = eng->dev_malloc(std::max<size_t>(n, 1) * sizeof(float));
     index_mem.push_back(p);
     return static_cast<float*>(p);
   }

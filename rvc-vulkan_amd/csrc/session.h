@@ -171,16 +171,14 @@ struct SessionBase {
   }
 
   uint16_t* upload16(const std::vector<uint16_t>& v) {
-    void* p = nullptr;
-    RVC_HIP(hipMalloc(&p, std::max<size_t>(v.size(), 8) * sizeof(uint16_t)));
+    void* p = eng->dev_malloc(std::max<size_t>(v.size(), 8) * sizeof(uint16_t));
     owned.push_back(p);
     if (!v.empty()) RVC_HIP(hipMemcpy(p, v.data(), v.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
     return static_cast<uint16_t*>(p);
   }
 
   float* upload(const std::vector<float>& v) {
-    void* p = nullptr;
-    RVC_HIP(hipMalloc(&p, std::max<size_t>(v.size(), 1) * sizeof(float)));
+    void* p = eng->dev_malloc(std::max<size_t>(v.size(), 1) * sizeof(float));
     owned.push_back(p);
     if (!v.empty()) RVC_HIP(hipMemcpy(p, v.data(), v.size() * sizeof(float), hipMemcpyHostToDevice));
     return static_cast<float*>(p);
@@ -198,8 +196,7 @@ struct SessionBase {
   unsigned* pq = nullptr;
   unsigned* persist_queue() {
     if (!pq) {
-      void* p = nullptr;
-      RVC_HIP(hipMalloc(&p, 16 * sizeof(unsigned)));
+      void* p = eng->dev_malloc(16 * sizeof(unsigned));
       owned.push_back(p);
       RVC_HIP(hipMemsetAsync(p, 0, 16 * sizeof(unsigned), eng->stream));
       pq = static_cast<unsigned*>(p);
@@ -216,12 +213,7 @@ struct SessionBase {
       RVC_HIP(hipFree(it->second.first));
       ws.erase(it);
     }
-    void* p = nullptr;
-    if (hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(float)) != hipSuccess) {
-      (void)hipGetLastError();
-      eng->trim_pool();
-      RVC_HIP(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(float)));
-    }
+    void* p = eng->dev_malloc(std::max<size_t>(n, 1) * sizeof(float));
     ws[name] = {static_cast<float*>(p), n};
     return static_cast<float*>(p);
   }

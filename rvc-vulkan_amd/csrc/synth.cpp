@@ -177,8 +177,7 @@ struct Synth : SessionBase {
   unsigned* errh = nullptr;
   void begin_ids() {
     if (!errw) {
-      void* p = nullptr;
-      RVC_HIP(hipMalloc(&p, 256));
+      void* p = eng->dev_malloc(256);
       owned.push_back(p);
       errw = static_cast<unsigned*>(p);
       RVC_HIP(hipHostMalloc((void**)&errh, sizeof(unsigned), hipHostMallocDefault));
