@@ -152,21 +152,21 @@ __global__ __launch_bounds__(64 * NW) void conv2d_split_kernel(Conv2dLaunch a, i
   for (int r = 0; r < 16; ++r)
     acc[r] *= buf_load4(srs, 4u * (unsigned)(co0 + 4 * half), 4 * ((r & 3) + 8 * (r >> 2))) * (1.f / sx);
   if (redo) {  // a NaN among the sums: this wave's channels again in fp32
-#pragma unroll 1
-    for (int q = 0; q < 16; ++q) {
-      const int co = co0 + 4 * half + (q & 3) + 8 * (q >> 2);
-      float v = 0.f;
-      for (int t = 0; t < T; ++t) {
-        const int h = pr + G.dh[t], w = pc + G.dw[t];
-        const bool in = h >= 0 && h < a.H && w >= 0 && w < a.W;
-        for (int ci = 16 * c_lo; ci < 16 * c_hi; ++ci)
-          v = fmaf(co < a.C_out ? G.w[((long long)t * a.C_in + ci) * a.w_ld + co] : 0.f,
-                   in ? xb[(long long)ci * a.xc + (long long)h * a.W + w] : 0.f, v);
-      }
-#pragma unroll
-      for (int z = 0; z < 16; ++z)
-        if (z == q) acc[z] = v;
-    }
+    floatx16 f[1][1];
+    const __amdgpu_buffer_rsrc_t frs = uniform_rsrc(G.w, 4u * (unsigned)(T * a.C_in * a.w_ld));
+    const unsigned fo = co0 + l32 < a.C_out ? 4u * (unsigned)(half * a.w_ld + co0 + l32) : kBufOut;
+    fp32_sums(
+        f, 16 * (c_hi - c_lo), T,
+        [&](float(&A)[1], int t, int c) {
+          A[0] = buf_load4(frs, fo, 4u * (unsigned)((t * a.C_in + 16 * c_lo + c) * a.w_ld));
+        },
+        [&](float(&B)[1], int t, int c) {
+          const __amdgpu_buffer_rsrc_t rs =
+              uniform_rsrc(xb + (long long)(16 * c_lo + c) * a.xc, xrow + 4u * (unsigned)(a.H * a.W));
+          const int h = pr + G.dh[t], w = pc + G.dw[t];
+          B[0] = buf_load4(rs, h >= 0 && h < a.H && w >= 0 && w < a.W ? half * xrow + 4u * (unsigned)(h * a.W + w) : kBufOut, 0);
+        });
+    acc = f[0][0];
   }
 
   // ---- partial tiles [wave][channel][point], added in wave order

@@ -1467,19 +1467,22 @@ void conv1x1_split_kernel(ConvLaunch a, int n_row, int n_col) {
     for (int r = 0; r < 16; ++r)
       acc[m][r] *= buf_load4(srs, 4u * (unsigned)(co0 + 4 * half), 4 * (m * 32 + (r & 3) + 8 * (r >> 2))) * (1.f / sx);
   if (redo) {  // this wave's channels again in fp32
-#pragma unroll 1
-    for (int q = 0; q < TM * 16; ++q) {
-      const int r = q & 15, co = co0 + 4 * half + (q >> 4) * 32 + (r & 3) + 8 * (r >> 2);
-      float v = 0.f;
-      for (int ci = 16 * s_lo; ci < 16 * s_hi; ++ci) {
-        float x = col < a.L_in ? xb[(long long)ci * a.xc + col] : 0.f;
-        if (ln) x = (x - ln_mu) * ln_rd;
-        v = fmaf(G.w[(long long)ci * a.w_ld + co], x, v);
-      }
+    floatx16 f[TM][1];
+    const __amdgpu_buffer_rsrc_t frs = uniform_rsrc(G.w, 4u * (unsigned)(C_in * a.w_ld));
+    const unsigned fo = 4u * (unsigned)(half * a.w_ld + co0 + l32);
+    const unsigned xf = col < a.L_in ? 4u * (unsigned)(half * (int)a.xc + col) : kBufOut;
+    fp32_sums(
+        f, 16 * (s_hi - s_lo), 1,
+        [&](float(&A)[TM], int, int c) {
 #pragma unroll
-      for (int z = 0; z < TM * 16; ++z)
-        if (z == q) acc[z / 16][z % 16] = v;
-    }
+          for (int m = 0; m < TM; ++m) A[m] = buf_load4(frs, fo + 128u * m, 4u * (unsigned)((16 * s_lo + c) * a.w_ld));
+        },
+        [&](float(&B)[1], int, int c) {
+          const float x = buf_load4(xrs, xf, 4u * (unsigned)((16 * s_lo + c) * (int)a.xc));
+          B[0] = ln ? (x - ln_mu) * ln_rd : x;
+        });
+#pragma unroll
+    for (int m = 0; m < TM; ++m) acc[m] = f[m][0];
   }
 #pragma unroll
   for (int m = 0; m < TM; ++m) {

@@ -23,8 +23,9 @@
 // bits to fp16's subnormals, a larger one overflows) it forms the tile again
 // with the power of two that puts that magnitude into [2^9, 2^10).
 // Infinities and NaN: every output such an input or weight reaches is NaN
-// here; a wave that finds a NaN among its sums forms them again in fp32 from
-// the fp32 weights, which gives what an fp32 convolution gives.
+// here; a wave that finds a NaN among its sums forms them again on the fp32
+// matrix cores from the fp32 weights (fp32_sums), which gives what an fp32
+// convolution gives.
 //
 // One workgroup forms a BM x BN tile, wave (wm, wn) a WM x WN part of it, over
 // chunks of 16 input channels.  A chunk's input window (BN + (K - 1) dil
@@ -276,23 +277,23 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
         for (int r = 0; r < 16; ++r) acc[m][n][r] = acc[m][n][r] * (sc[r] * inv);
     }
     if (redo) {
-#pragma unroll 1
-      for (int q = 0; q < TM * TN * 16; ++q) {
-        const int r = q & 15, n = (q >> 4) % TN, m = (q >> 4) / TN;
-        const int co = co_l + m * 32 + (r & 3) + 8 * (r >> 2);
-        const int i = i0 + wn * WN + n * 32 + l32;
-        float v = 0.f;
-        for (int ci = 0; ci < a.C_in; ++ci)
-          for (int k = 0; k < K; ++k) {
-            const int t = i * S + G.in_off + k * dil;
-            float x = t >= 0 && t < a.L_in ? xb[(long long)ci * a.xc + t] : 0.f;
-            if (a.in_act == ACT_LEAKY) x = leaky(x, a.in_slope);
-            v = fmaf(G.w[((long long)k * a.C_in + ci) * a.w_ld + co], x, v);
-          }
+      const __amdgpu_buffer_rsrc_t frs = uniform_rsrc(G.w, 4u * (unsigned)(K * a.C_in * a.w_ld));
+      const unsigned fo = 4u * (unsigned)(half * a.w_ld + co0 + wm * WM + l32);
+      fp32_sums(
+          acc, a.C_in, K,
+          [&](float(&A)[TM], int k, int c) {
 #pragma unroll
-        for (int z = 0; z < TM * TN * 16; ++z)
-          if (z == q) acc[z / (TN * 16)][(z / 16) % TN][z % 16] = v;
-      }
+            for (int m = 0; m < TM; ++m) A[m] = buf_load4(frs, fo + 128u * m, 4u * (unsigned)((k * a.C_in + c) * a.w_ld));
+          },
+          [&](float(&B)[TN], int k, int c) {
+            const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(xb + (long long)c * a.xc, 4u * (unsigned)((int)a.xc + a.L_in));
+#pragma unroll
+            for (int n = 0; n < TN; ++n) {
+              const int t = (i0 + wn * WN + n * 32 + l32) * S + G.in_off + k * dil;
+              const float v = buf_load4(rs, t >= 0 && t < a.L_in ? 4u * (unsigned)(half * (int)a.xc + t) : kBufOut, 0);
+              B[n] = a.in_act == ACT_LEAKY ? leaky_mma(v, a.in_slope) : v;
+            }
+          });
     }
   }
 

@@ -17,8 +17,9 @@
 // conv2's padding wants them.
 //
 // The input's scale is that of conv_split.hip, and so is the intermediate's,
-// which is still in registers when its tile's largest value is known.  NaN sums are formed again in fp32 in both convs, the second
-// from the two parts in LDS (an infinity is stored as (inf, 0)).
+// which is still in registers when its tile's largest value is known.  A wave
+// with NaN sums forms them again on the fp32 matrix cores in both convs, the
+// second from the two parts in LDS (an infinity is stored as (inf, 0)).
 //
 // 40k, 1000 frames, ms of a stage's six convs, two launches -> fused: C = 128
 // 1.20 -> 1.19 (half the launches), C = 64 0.78 -> 0.69, C = 32 0.60 -> 0.45
@@ -216,16 +217,26 @@ void resblock_pair_kernel(PairLaunch a) {
     }
     return (bool)__any(bad);
   };
-  // every sum of the wave again, from dot(row, column)
-  auto form_again = [&](auto dot) {
-#pragma unroll 1
-    for (int q = 0; q < TM * TN * 16; ++q) {
-      const int r = q & 15, n = (q >> 4) % TN, m = (q >> 4) / TN;
-      const float v = dot(co_l + m * 32 + (r & 3) + 8 * (r >> 2), wn * WN + n * 32 + l32);
+  // the wave's sums again in fp32, from weights [K][C][C] and x(B, k, c)
+  // (fp32_sums), and their bias
+  auto form_again = [&](const float* w, const float* bias, auto x) {
+    const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(w, 4u * (unsigned)(K * C * C)), rb = uniform_rsrc(bias, 4u * C);
+    const unsigned fo = 4u * (unsigned)(half * C + wm * WM + l32);
+    fp32_sums(
+        acc, C, K,
+        [&](float(&A)[TM], int k, int c) {
 #pragma unroll
-      for (int z = 0; z < TM * TN * 16; ++z)
-        if (z == q) acc[z / (TN * 16)][(z / 16) % TN][z % 16] = v;
-    }
+          for (int m = 0; m < TM; ++m) A[m] = buf_load4(rs, fo + 128u * m, 4u * (unsigned)((k * C + c) * C));
+        },
+        x);
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float t = buf_load4(rb, 4u * (unsigned)co_l, 4 * (m * 32 + (r & 3) + 8 * (r >> 2)));
+#pragma unroll
+        for (int n = 0; n < TN; ++n) acc[m][n][r] += t;
+      }
   };
 
   // ---- conv1 over the BN intermediate columns
@@ -251,15 +262,13 @@ void resblock_pair_kernel(PairLaunch a) {
   const bool redo1 = !BF && any_nan(BN);
   finish(G.w1.sc, 1.f / sx, G.b1);
   if (redo1)
-    form_again([&](int co, int col) {
-      float v = 0.f;
-      for (int ci = 0; ci < C; ++ci)
-        for (int k = 0; k < K; ++k) {
-          const int t = x0 + col + k * dil;
-          const float x = t >= 0 && t < L ? leaky(xb[(long long)ci * L + t], a.slope) : 0.f;
-          v = fmaf(G.f1[((long long)k * C + ci) * C + co], x, v);
-        }
-      return v + G.b1[co];
+    form_again(G.f1, G.b1, [&](float(&B)[TN], int k, int c) {
+      const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(xb + (long long)c * L, 8u * (unsigned)L);
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        const int t = x0 + wn * WN + n * 32 + l32 + k * dil;
+        B[n] = leaky_mma(buf_load4(rs, t >= 0 && t < L ? 4u * (unsigned)(half * L + t) : kBufOut, 0), a.slope);
+      }
     });
 
   // ---- leaky ReLU, zero outside the signal, scale, split to LDS
@@ -333,18 +342,18 @@ void resblock_pair_kernel(PairLaunch a) {
   const int cols = min(BO, L - o0);
   const bool redo2 = !BF && any_nan(cols);
   finish(G.w2.sc, 1.f / sy, G.b2);
-  if (redo2)
-    form_again([&](int co, int col) {
-      float v = 0.f;
-      const float inv = 1.f / sy;
-      for (int ci = 0; ci < C; ++ci)
-        for (int k = 0; k < K; ++k) {
-          const _Float16* p = reinterpret_cast<const _Float16*>(sm + (ci / 8) * YW + min(col + k, YW - 1)) + ci % 8;
-          const float y = ((float)p[0] + (float)p[(C / 8) * YW * 8]) * inv;
-          v = fmaf(G.f2[((long long)k * C + ci) * C + co], y, v);
-        }
-      return v + G.b2[co];
+  if (redo2) {
+    const float inv = 1.f / sy;
+    form_again(G.f2, G.b2, [&](float(&B)[TN], int k, int c) {
+      const int ci = c + half;
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        const int col = wn * WN + n * 32 + l32 + k;
+        const _Float16* p = reinterpret_cast<const _Float16*>(sm + (ci / 8) * YW + col) + ci % 8;
+        B[n] = ((float)p[0] + (float)p[(C / 8) * YW * 8]) * inv;
+      }
     });
+  }
   const __amdgpu_buffer_rsrc_t rrs = uniform_rsrc(xb, 4u * (unsigned)(C * L));
   const __amdgpu_buffer_rsrc_t ors = uniform_rsrc(G.out + (long long)b * C * L, 4u * (unsigned)(C * L));
 #pragma unroll

@@ -31,12 +31,16 @@ __device__ __forceinline__ float buf_load4(__amdgpu_buffer_rsrc_t r, unsigned vo
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 // leaky ReLU for slopes in [0, 1]: max(v, v slope), as one instruction each
-// (fmaxf quiets its operands first)
+// (fmaxf quiets its operands first).  Never straight into or out of an MFMA: the
+// compiler does not see the asm as the VALU instruction it is, and leaves out the
+// wait states between the two.
 __device__ __forceinline__ float leaky(float v, float slope) {
   float r;
   asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(v), "v"(v * slope));
   return r;
 }
+// the same for operands of an MFMA
+__device__ __forceinline__ float leaky_mma(float v, float slope) { return v < 0.f ? v * slope : v; }
 // max(m, |a|, |b|)
 __device__ __forceinline__ float max3_abs(float m, float a, float b) {
   asm("v_max3_f32 %0, %0, abs(%1), abs(%2)" : "+v"(m) : "v"(a), "v"(b));
@@ -86,6 +90,38 @@ __device__ __forceinline__ void stage_unit(float (&v)[8], float sx, float& vmax,
     dst[0] = h;
     dst[part] = l;
   }
+}
+// A wave's 32 TM x 32 TN sums on the fp32 matrix cores, from where the operands
+// lie in fp32, C channels (a multiple of 8) by K taps: the sums that a split
+// cannot form.  w(A, k, c) fills A[m] with row 32 m + lane % 32's weight of
+// channel c + lane / 32 and tap k, x(B, k, c) B[n] with column 32 n + lane % 32's
+// input.
+template <int TM, int TN, class W, class X>
+__device__ __forceinline__ void fp32_sums(floatx16 (&acc)[TM][TN], int C, int K, W w, X x) {
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < K; ++k)
+#pragma unroll 1
+    for (int c = 0; c < C; c += 8) {
+      float A[4][TM], B[4][TN];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        w(A[u], k, c + 2 * u);
+        x(B[u], k, c + 2 * u);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int n = 0; n < TN; ++n)
+            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[u][m], B[u][n], acc[m][n], 0, 0, 0);
+    }
 }
 template <int TM>
 __device__ __forceinline__ void swap_sets(uint4 (&a)[2][TM], uint4 (&b)[2][TM]) {
