@@ -1365,8 +1365,9 @@ __global__ __launch_bounds__(64 * NW) void conv_small_kernel(ConvLaunch a) {
 // channels a chunk behind two barriers, ran at a quarter of its time without
 // its MFMAs.
 //
-// The input's scale is per wave (its partial sums are unscaled before they are
-// added); its LayerNorm from the producer's column statistics (ln_stat) is
+// The input's scale is its column's in the wave's run of channels (the partial
+// sums are unscaled before they are added): what a column gives does not hang on
+// its neighbours.  Its LayerNorm from the producer's column statistics (ln_stat) is
 // applied on the way in.  The row tiles go round the XCDs, so each weight is
 // read into one L2.  What remains is latency: a wave's three to twelve pairs of
 // steps, the column statistics in front and the epilogue behind.
@@ -1446,12 +1447,11 @@ void conv1x1_split_kernel(ConvLaunch a, int n_row, int n_col) {
       if (s + 2 < s_hi) step(1);
     }
     if (again) break;
-    float m = xmax;
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
-    m = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m)));
-    if (m == 0.f || (m >= kXMin * kScaleX && m <= kXMax * kScaleX) || __builtin_isinf(m)) break;
-    sx = pow2_scale(m * (1.f / kScaleX));
+    // a column's largest magnitude; the sums of an infinite one are NaN at any scale
+    const float m = fmaxf(xmax, __shfl_xor(xmax, 32));
+    const bool fits = split_holds(m) || __builtin_isinf(m);
+    if (__all(fits)) break;
+    sx = fits ? kScaleX : pow2_scale(m * (1.f / kScaleX));
     load(s_lo, 0);
   }
   float nan = 0.f;
@@ -1459,14 +1459,14 @@ void conv1x1_split_kernel(ConvLaunch a, int n_row, int n_col) {
   for (int m = 0; m < TM; ++m)
 #pragma unroll
     for (int r = 0; r < 16; ++r) nan = fmaf(acc[m][r], 0.f, nan);
-  const bool redo = __any(nan != nan && col < a.L_in);
+  const bool bad = nan != nan && col < a.L_in;
   const __amdgpu_buffer_rsrc_t srs = uniform_rsrc(G.wsc, 4u * (unsigned)a.C_out);
 #pragma unroll
   for (int m = 0; m < TM; ++m)
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       acc[m][r] *= buf_load4(srs, 4u * (unsigned)(co0 + 4 * half), 4 * (m * 32 + (r & 3) + 8 * (r >> 2))) * (1.f / sx);
-  if (redo) {  // this wave's channels again in fp32
+  if (__any(bad)) {  // this wave's channels again in fp32
     floatx16 f[TM][1];
     const __amdgpu_buffer_rsrc_t frs = uniform_rsrc(G.w, 4u * (unsigned)(C_in * a.w_ld));
     const unsigned fo = 4u * (unsigned)(half * a.w_ld + co0 + l32);
@@ -1482,7 +1482,9 @@ void conv1x1_split_kernel(ConvLaunch a, int n_row, int n_col) {
           B[0] = ln ? (x - ln_mu) * ln_rd : x;
         });
 #pragma unroll
-    for (int m = 0; m < TM; ++m) acc[m] = f[m][0];
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[m][r] = bad ? f[m][0][r] : acc[m][r];
   }
 #pragma unroll
   for (int m = 0; m < TM; ++m) {

@@ -15,6 +15,12 @@ typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 
 constexpr float kScaleX = 64.f;                 // the inputs' usual scale
 constexpr float kXMin = 0x1p-6f, kXMax = 960.f;  // the magnitudes it serves
+// whether a largest magnitude m, scaled, lies where the two parts hold what the
+// sums need: 0, or from where fp16's subnormals cost less than 2^-24 of it up to
+// where fp16 ends.  Infinities and NaN do not.
+__device__ __forceinline__ bool split_holds(float m) {
+  return m == 0.f || (m >= kXMin * kScaleX && m <= kXMax * kScaleX);
+}
 
 // one product of two operands: 8 channels of a row and of a column per lane
 template <bool BF>

@@ -55,3 +55,19 @@ def test_infinite_and_nan_rows_are_never_found():
     w[17, 3], w[50, 4] = np.nan, np.inf
     scores, rows = _search(w, q)
     assert np.isfinite(scores).all() and not np.isin(rows, (17, 50)).any()
+
+
+@pytest.mark.parametrize("exponent", [-60, -20, 12, 20, 60])
+def test_a_query_does_not_hang_on_its_neighbours(exponent):
+    """Queries of another size, an infinite and a NaN one share tiles with the
+    rest, whose distances stay bit for bit what they are without them."""
+    v, q = _case(300, 70, 768, 7)
+    scores, rows = _search(v, q)
+    other = q.copy()
+    other[5::16] *= np.float32(2.0) ** exponent
+    other[9, 3], other[41, 700] = np.nan, np.inf
+    keep = np.ones(len(q), bool)
+    keep[5::16] = keep[[9, 41]] = False
+    got, at = _search(v, other)
+    np.testing.assert_array_equal(got[keep], scores[keep])
+    np.testing.assert_array_equal(at[keep], rows[keep])
