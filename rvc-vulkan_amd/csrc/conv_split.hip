@@ -18,14 +18,18 @@
 // launches at 190 - 220 TFLOP/s of fp32 products, error 1.6e-6.)
 //
 // Range: weights are scaled per output row to a largest value in [2^9, 2^10),
-// inputs by 2^6, all exactly (powers of two).  A workgroup keeps the largest
-// input magnitude of its window; outside [2^-6, 2^9.9] (a smaller one loses
-// bits to fp16's subnormals, a larger one overflows) it forms the tile again
-// with the power of two that puts that magnitude into [2^9, 2^10).
-// Infinities and NaN: every output such an input or weight reaches is NaN
-// here; a wave that finds a NaN among its sums forms them again on the fp32
-// matrix cores from the fp32 weights (fp32_sums), which gives what an fp32
-// convolution gives.
+// inputs by 2^6, all exactly (powers of two).  At that scale the two parts hold
+// a column whose largest input, of all channels and taps, is in [2^-6, 2^9.9]: a
+// smaller one loses bits to fp16's subnormals, a larger one overflows.  A
+// workgroup keeps the largest magnitude of each unit of 8 channels and a column
+// that it stages.  Where none of them fits, it forms the tile again with the
+// power of two that puts the largest into [2^14, 2^15); where some do, it looks
+// at each output's own columns, and those that do not fit (an infinity among
+// them, or a NaN among the sums) are formed on the fp32 matrix cores from the
+// fp32 weights (fp32_sums), which gives what an fp32 convolution gives.  So an
+// output has fp32's precision and reach whatever else is in its tile, as far
+// as its inputs go; within an output's own inputs, channels or taps far below
+// the largest keep 2^-31 absolute (2^-40 of the row's largest weight).
 //
 // One workgroup forms a BM x BN tile, wave (wm, wn) a WM x WN part of it, over
 // chunks of 16 input channels.  A chunk's input window (BN + (K - 1) dil
@@ -103,6 +107,7 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
 
   extern __shared__ uint4 sm[];  // [2 buffers][2][2][XW]
   __shared__ float wmax[C::NW];
+  __shared__ unsigned vote[C::NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave % C::NWM, wn = wave / C::NWM;
   const int half = lane >> 5, l32 = lane & 31;
@@ -131,7 +136,7 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) xv[e][j] = buf_load4(rs, xo[e], j * xrow);
   };
-  float sx = kScaleX, xmax = 0.f;
+  float sx = kScaleX, xm[XPT];  // each unit's largest magnitude, scaled
   auto lstore_as = [&](int buf, auto act) __attribute__((always_inline)) {
     uint4* xs = sm + buf * 4 * XW;
 #pragma unroll
@@ -140,7 +145,7 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
       float v[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = decltype(act)::value ? leaky(xv[e][j], a.in_slope) : xv[e][j];
-      stage_unit<BF>(v, sx, xmax, xs + xu[e], 2 * XW);
+      stage_unit<BF>(v, sx, xm[e], xs + xu[e], 2 * XW);
     }
   };
   auto lstore = [&](int buf) __attribute__((always_inline)) {
@@ -170,6 +175,7 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
         acc[m][n] = mma16<BF>(A[m], B[n], acc[m][n]);
   };
 
+  bool mixed = false;  // some units lie outside the split's range
   for (bool again = false;; again = true) {
 #pragma unroll
     for (int m = 0; m < TM; ++m)
@@ -177,6 +183,8 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
       for (int n = 0; n < TN; ++n)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+#pragma unroll
+    for (int e = 0; e < XPT; ++e) xm[e] = 0.f;
     gload(0);
     // last: the last step's weights; next: the ones to load
     const unsigned last = (unsigned)(nchunk * K - 1) * 2u * wpart;
@@ -238,32 +246,49 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
       if (more) lstore((c & 1) ^ 1);
       __syncthreads();
     }
-    if (BF || again) break;
-    // the window's largest magnitude (scaled by kScaleX): the tile again with
-    // a scale of its own where fp16's range does not hold it
-    float m = xmax;
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
-    if (lane == 0) wmax[wave] = m;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < C::NW; ++w) m = fmaxf(m, wmax[w]);
-    m = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m)));
-    if (m == 0.f || (m >= kXMin * kScaleX && m <= kXMax * kScaleX) || __builtin_isinf(m)) break;
-    sx = pow2_scale(m * (1.f / kScaleX));
+    if (BF) break;
+    float top;
+    const unsigned f = block_or<C::NW>(range_bits(xm, 1.f, top), vote);
+    mixed = f & 1u;
+    if (!mixed || again || (f & 2u)) break;
+    top = block_max<C::NW>(top, wmax);
+    if (top == 0.f) break;  // infinities and zeros
+    sx = pow2_scale(top * (1.f / kScaleX));
   }
 
   const int co_l = co0 + wm * WM + 4 * half;
   if constexpr (!BF) {
-    // ---- a NaN among the sums: form them again in fp32
-    float nan = 0.f;
+    // ---- the lane's columns that the split does not hold (bit n)
+    unsigned bad = 0;
+    if (mixed) {
+      unsigned* cm = reinterpret_cast<unsigned*>(sm);  // a column's largest magnitude; every wave is past its operands
+      for (int u = tid; u < XW; u += NT) cm[u] = 0u;
+      __syncthreads();
 #pragma unroll
-    for (int m = 0; m < TM; ++m)
+      for (int e = 0; e < XPT; ++e)
+        if (xu[e] >= 0) atomicMax(cm + (xu[e] < XW ? xu[e] : xu[e] - XW), __builtin_bit_cast(unsigned, xm[e]));
+      __syncthreads();
 #pragma unroll
-      for (int n = 0; n < TN; ++n)
+      for (int n = 0; n < TN; ++n) {
+        const unsigned* p = cm + wn * WN + n * 32 + l32;
+        unsigned t = 0;
+        for (int k = 0; k < K; ++k) {
+          t = max(t, *p);
+          if (k + 1 < K) p += S == 2 ? ((k & 1) ? -BN : BN + 1) : dil;
+        }
+        if (!split_holds(__builtin_bit_cast(float, t))) bad |= 1u << n;
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      float nan = 0.f;
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int r = 0; r < 16; ++r) nan = fmaf(acc[m][n][r], 0.f, nan);
-    const bool redo = __any(nan != nan);
+      if (nan != nan) bad |= 1u << n;
+      if (i0 + wn * WN + n * 32 + l32 >= n_out) bad &= ~(1u << n);
+    }
     const __amdgpu_buffer_rsrc_t srs = uniform_rsrc(G.wsc, 4u * (unsigned)a.C_out);
     const float inv = 1.f / sx;
 #pragma unroll
@@ -276,11 +301,12 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[m][n][r] = acc[m][n][r] * (sc[r] * inv);
     }
-    if (redo) {
+    if (__any(bad != 0u)) {
+      floatx16 f[TM][TN];
       const __amdgpu_buffer_rsrc_t frs = uniform_rsrc(G.w, 4u * (unsigned)(K * a.C_in * a.w_ld));
       const unsigned fo = 4u * (unsigned)(half * a.w_ld + co0 + wm * WM + l32);
       fp32_sums(
-          acc, a.C_in, K,
+          f, a.C_in, K,
           [&](float(&A)[TM], int k, int c) {
 #pragma unroll
             for (int m = 0; m < TM; ++m) A[m] = buf_load4(frs, fo + 128u * m, 4u * (unsigned)((k * a.C_in + c) * a.w_ld));
@@ -294,6 +320,12 @@ void conv1d_split_kernel(ConvLaunch a, int n_tx, int n_ty) {
               B[n] = a.in_act == ACT_LEAKY ? leaky_mma(v, a.in_slope) : v;
             }
           });
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+#pragma unroll
+        for (int n = 0; n < TN; ++n)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[m][n][r] = bad >> n & 1u ? f[m][n][r] : acc[m][n][r];
     }
   }
 
@@ -405,7 +437,7 @@ void launch_conv1d_split(const ConvLaunch& a, hipStream_t s) {
   if (n == 0) return;
   // The widest tile that leaves one batch item 400 workgroups; never by B, so
   // that a batch equals its items bit for bit also where a tile's own scale
-  // shows.  C = 256 at 10 000 columns (40k stage 0, 1000 frames, ms
+  // or its fp32 sums show.  C = 256 at 10 000 columns (40k stage 0, 1000 frames, ms
   // of its six launches): 64 x 128 0.60, 128 x 128 0.65, 64 x 256 0.76 (the fp32
   // matrix cores: 1.42).
   // tiles of one batch item

@@ -22,6 +22,45 @@ __device__ __forceinline__ bool split_holds(float m) {
   return m == 0.f || (m >= kXMin * kScaleX && m <= kXMax * kScaleX);
 }
 
+// the OR over the waves of a workgroup of its threads' low two bits; one barrier,
+// slot: NW words that no wave still reads from an earlier call
+template <int NW>
+__device__ __forceinline__ unsigned block_or(unsigned bits, unsigned* slot) {
+  const unsigned v = (__any(bits & 1u) ? 1u : 0u) | (__any(bits & 2u) ? 2u : 0u);
+  if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = v;
+  __syncthreads();
+  unsigned f = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) f |= slot[w];
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)f);
+}
+// the largest m over a workgroup; two barriers
+template <int NW>
+__device__ __forceinline__ float block_max(float m, float* slot) {
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+  if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) m = fmaxf(m, slot[w]);
+  __syncthreads();
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m)));
+}
+// largest magnitudes m[i]: bit 0 where one does not lie in the split's range,
+// bit 1 where one does and is not 0; top: the largest finite one
+template <int N>
+__device__ __forceinline__ unsigned range_bits(const float (&m)[N], float scale, float& top) {
+  unsigned f = 0;
+  top = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float v = m[i] * scale;
+    f |= split_holds(v) ? (v > 0.f ? 2u : 0u) : 1u;
+    top = m[i] < __builtin_inff() ? fmaxf(top, m[i]) : top;
+  }
+  return f;
+}
+
 // one product of two operands: 8 channels of a row and of a column per lane
 template <bool BF>
 __device__ __forceinline__ floatx16 mma16(uint4 w, uint4 x, floatx16 c) {
@@ -71,11 +110,11 @@ __device__ __forceinline__ void split2_inf(float a, float b, unsigned& h, unsign
   h = __builtin_bit_cast(unsigned, hv);
   l = __builtin_bit_cast(unsigned, __builtin_convertvector(r, halfx2));
 }
-// the power of two that moves m (finite, above 0) into [2^9, 2^10), within the
-// normal floats on both sides of 1
+// the power of two that moves m (finite, above 0) into [2^14, 2^15), within the
+// normal floats on both sides of 1: what lies up to 2^14 below it is held too
 __device__ __forceinline__ float pow2_scale(float m) {
   const int e = (int)(__builtin_bit_cast(unsigned, m) >> 23) - 127;
-  return __builtin_bit_cast(float, (unsigned)(min(max(9 - e, -126), 126) + 127) << 23);
+  return __builtin_bit_cast(float, (unsigned)(min(max(14 - e, -126), 126) + 127) << 23);
 }
 // eight channels of one column to LDS: their fp16 parts of v * sx at dst and
 // dst + part, largest magnitude to vmax; or (BF) their bf16 at dst

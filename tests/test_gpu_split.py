@@ -91,6 +91,28 @@ def test_infinity_reaches_what_it_reaches_in_fp32(decoders, name):
     assert np.isnan(got[np.isnan(want)]).all()
 
 
+@pytest.mark.parametrize("name", ["plain"])
+@pytest.mark.parametrize("exponent", [24, 60, 100])
+def test_a_spike_takes_nothing_from_its_neighbours(decoders, name, exponent):
+    """The samples that frames of huge or infinite z do not reach share tiles with
+    those they do, and keep their fp32 precision: what is computed twice, with
+    and without the spikes, differs by the error of two such computations."""
+    geom, _, hip, ref = decoders[name]
+    d = syn.make_dec_inputs(geom, 700, seed=9)
+    z, zi = d["z"].copy(), d["z"].copy()
+    z[0, :, 70::160] = np.float32(2.0) ** exponent
+    zi[0, :, 70::160] = np.inf
+    with nn_ref.conv_formulation("taps"), np.errstate(all="ignore"):
+        reach = ref.forward(zi, d["f0"], d["g"], d["ns"])
+        clean = ref.forward(d["z"], d["f0"], d["g"], d["ns"])
+    fine = np.abs(reach - clean) < 1e-6
+    assert 0.1 < fine.mean() < 0.9
+    want = hip.dec.forward(d["z"], d["f0"], d["g"], d["ns"])
+    for x in (z, zi):
+        got = hip.dec.forward(x, d["f0"], d["g"], d["ns"])
+        assert rel_l2(got[fine], want[fine]) < 3e-6
+
+
 @pytest.mark.parametrize("name,P", [("fused", P) for P in (1, 17, 64, 129, 2100, 8400, 16900)] +
                          [("plain", P) for P in (1, 33, 1601, 4300)])
 def test_bf16_tile_edges(decoders, name, P):
