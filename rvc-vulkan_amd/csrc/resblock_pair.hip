@@ -17,9 +17,10 @@
 // conv2's padding wants them.
 //
 // The input's scale is that of conv_split.hip, and so is the intermediate's,
-// which is still in registers when its tile's largest value is known.  A wave
-// with NaN sums forms them again on the fp32 matrix cores in both convs, the
-// second from the two parts in LDS (an infinity is stored as (inf, 0)).
+// which is still in registers when its columns' largest values are known.  What
+// the scales do not hold takes the fp32 matrix cores (fp32_sums): columns of
+// the intermediate from x, and outputs whose intermediate columns do not fit
+// from an fp32 intermediate, which has just the two parts' room in LDS.
 //
 // 40k, 1000 frames, ms of a stage's six convs, two launches -> fused: C = 128
 // 1.20 -> 1.19 (half the launches), C = 64 0.78 -> 0.69, C = 32 0.60 -> 0.45
@@ -49,6 +50,7 @@ void resblock_pair_kernel(PairLaunch a) {
   constexpr int XPT = (XU * (BN + kConvHaloMax) + NT - 1) / NT;
   constexpr int nchunk = C / CH, PARTS = BF ? 1 : 2;
   constexpr unsigned wpart = 1024u * NRB;
+  constexpr int YS = BN + kConvTapsMax - 1;  // row length of an fp32 intermediate in LDS
   int gi = 0, lin = blockIdx.x;
   while (gi + 1 < a.n && lin >= a.g[gi].tiles * a.B) {
     lin -= a.g[gi].tiles * a.B;
@@ -65,6 +67,7 @@ void resblock_pair_kernel(PairLaunch a) {
 
   extern __shared__ uint4 sm[];  // [2 buffers][2 parts][2][XW], then [2 parts][C / 8][YW]
   __shared__ float wmax[NW];
+  __shared__ unsigned vote[3][NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave % NWM, wn = wave / NWM;
   const int half = lane >> 5, l32 = lane & 31;
@@ -91,7 +94,7 @@ void resblock_pair_kernel(PairLaunch a) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) xv[e][j] = buf_load4(rs, xo[e], 4u * (unsigned)(j * L));
   };
-  float sx = kScaleX, xmax = 0.f;
+  float sx = kScaleX, xm[XPT];  // each unit's largest magnitude, scaled
   auto lstore = [&](int buf) __attribute__((always_inline)) {
     uint4* xs = sm + buf * 4 * XW;
 #pragma unroll
@@ -100,20 +103,9 @@ void resblock_pair_kernel(PairLaunch a) {
       float v[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = leaky(xv[e][j], a.slope);
-      stage_unit<BF>(v, sx, xmax, xs + xu[e], 2 * XW);
+      stage_unit<BF>(v, sx, xm[e], xs + xu[e], 2 * XW);
     }
   };
-  auto block_max = [&](float m) {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
-    if (lane == 0) wmax[wave] = m;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < NW; ++w) m = fmaxf(m, wmax[w]);
-    __syncthreads();
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m)));
-  };
-
   const unsigned wvo = 16u * (unsigned)lane + 1024u * (unsigned)(wm * TM);
   const unsigned wbytes = (unsigned)(nchunk * K) * 2u * wpart;
   uint4 Ah[2][TM], Al[2][TM], Bh[TN], Bl[TN];  // the weights of the current step and of the next one
@@ -203,9 +195,9 @@ void resblock_pair_kernel(PairLaunch a) {
         for (int r = 0; r < 16; ++r) acc[m][n][r] = fmaf(acc[m][n][r], s[r], t[r]);
     }
   };
-  // whether this wave holds a NaN among the columns below `cols`
-  auto any_nan = [&](int cols) {
-    bool bad = false;
+  // bit n: the lane's sums of column block n hold a NaN
+  auto nan_bits = [&] {
+    unsigned bits = 0;
 #pragma unroll
     for (int n = 0; n < TN; ++n) {
       float nan = 0.f;
@@ -213,17 +205,31 @@ void resblock_pair_kernel(PairLaunch a) {
       for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int r = 0; r < 16; ++r) nan = fmaf(acc[m][n][r], 0.f, nan);
-      bad |= nan != nan && wn * WN + n * 32 + l32 < cols;
+      if (nan != nan) bits |= 1u << n;
     }
-    return (bool)__any(bad);
+    return bits;
   };
-  // the wave's sums again in fp32, from weights [K][C][C] and x(B, k, c)
-  // (fp32_sums), and their bias
-  auto form_again = [&](const float* w, const float* bias, auto x) {
+  // bit n: the lane's column block n has a column among the K from p on, `step`
+  // apart, whose largest magnitude (bits) the split does not hold at `scale`
+  auto unfit_bits = [&](const unsigned* cm, int step, float scale) {
+    unsigned bits = 0;
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      const unsigned* p = cm + wn * WN + n * 32 + l32;
+      unsigned t = 0;
+      for (int k = 0; k < K; ++k) t = max(t, p[k * step]);
+      if (!split_holds(__builtin_bit_cast(float, t) * scale)) bits |= 1u << n;
+    }
+    return bits;
+  };
+  // the lane's column blocks of `bits` again in fp32, from weights [K][C][C] and
+  // x(B, k, c) (fp32_sums), and their bias; every lane of the wave calls it
+  auto form_again = [&](unsigned bits, const float* w, const float* bias, auto x) {
+    floatx16 f[TM][TN];
     const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(w, 4u * (unsigned)(K * C * C)), rb = uniform_rsrc(bias, 4u * C);
     const unsigned fo = 4u * (unsigned)(half * C + wm * WM + l32);
     fp32_sums(
-        acc, C, K,
+        f, C, K,
         [&](float(&A)[TM], int k, int c) {
 #pragma unroll
           for (int m = 0; m < TM; ++m) A[m] = buf_load4(rs, fo + 128u * m, 4u * (unsigned)((k * C + c) * C));
@@ -235,14 +241,37 @@ void resblock_pair_kernel(PairLaunch a) {
       for (int r = 0; r < 16; ++r) {
         const float t = buf_load4(rb, 4u * (unsigned)co_l, 4 * (m * 32 + (r & 3) + 8 * (r >> 2)));
 #pragma unroll
-        for (int n = 0; n < TN; ++n) acc[m][n][r] += t;
+        for (int n = 0; n < TN; ++n) acc[m][n][r] = bits >> n & 1u ? f[m][n][r] + t : acc[m][n][r];
+      }
+  };
+  // outputs of the lane's column blocks of `bits`, with the residual
+  const int cols = min(BO, L - o0);
+  auto store = [&](unsigned bits) {
+    const __amdgpu_buffer_rsrc_t rrs = uniform_rsrc(xb, 4u * (unsigned)(C * L));
+    const __amdgpu_buffer_rsrc_t ors = uniform_rsrc(G.out + (long long)b * C * L, 4u * (unsigned)(C * L));
+#pragma unroll
+    for (int m = 0; m < TM; ++m)
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        const int col = wn * WN + n * 32 + l32;
+        const unsigned oo = col < cols && (bits >> n & 1u) ? 4u * (unsigned)(co_l * L + o0 + col) : kBufOut;
+        float pre[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) pre[r] = buf_load4(rrs, oo, 4 * (m * 32 + (r & 3) + 8 * (r >> 2)) * L);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[m][n][r] + pre[r]), ors, oo,
+                                                4 * (m * 32 + (r & 3) + 8 * (r >> 2)) * L, 0);
       }
   };
 
   // ---- conv1 over the BN intermediate columns
   const __amdgpu_buffer_rsrc_t w1 = uniform_rsrc(G.w1.w, wbytes);
+  bool mixed = false;  // some units lie outside the split's range
   for (bool again = false;; again = true) {
     zero();
+#pragma unroll
+    for (int e = 0; e < XPT; ++e) xm[e] = 0.f;
     gload(0);
     first(w1);
     lstore(0);
@@ -254,15 +283,34 @@ void resblock_pair_kernel(PairLaunch a) {
       if (more) lstore((c & 1) ^ 1);
       __syncthreads();
     }
-    if (BF || again) break;
-    const float m = block_max(xmax);
-    if (m == 0.f || (m >= kXMin * kScaleX && m <= kXMax * kScaleX) || __builtin_isinf(m)) break;
-    sx = pow2_scale(m * (1.f / kScaleX));
+    if (BF) break;
+    float top;
+    const unsigned f = block_or<NW>(range_bits(xm, 1.f, top), vote[0]);
+    mixed = f & 1u;
+    if (!mixed || again || (f & 2u)) break;
+    top = block_max<NW>(top, wmax);
+    if (top == 0.f) break;  // infinities and zeros
+    sx = pow2_scale(top * (1.f / kScaleX));
   }
-  const bool redo1 = !BF && any_nan(BN);
+  unsigned bad = 0;  // the lane's intermediate columns that the split does not hold
+  if constexpr (!BF) {
+    if (mixed) {
+      unsigned* cm = reinterpret_cast<unsigned*>(sm);  // a column's largest magnitude; every wave is past its operands
+      for (int u = tid; u < XW; u += NT) cm[u] = 0u;
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < XPT; ++e)
+        if (xu[e] >= 0) atomicMax(cm + (xu[e] < XW ? xu[e] : xu[e] - XW), __builtin_bit_cast(unsigned, xm[e]));
+      __syncthreads();
+      bad = unfit_bits(cm, dil, 1.f);
+      __syncthreads();  // the room is free again
+    }
+    bad |= nan_bits();
+  }
   finish(G.w1.sc, 1.f / sx, G.b1);
-  if (redo1)
-    form_again(G.f1, G.b1, [&](float(&B)[TN], int k, int c) {
+  const bool again1 = __any(bad != 0u);
+  if (again1)
+    form_again(bad, G.f1, G.b1, [&](float(&B)[TN], int k, int c) {
       const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(xb + (long long)c * L, 8u * (unsigned)L);
 #pragma unroll
       for (int n = 0; n < TN; ++n) {
@@ -272,39 +320,86 @@ void resblock_pair_kernel(PairLaunch a) {
     });
 
   // ---- leaky ReLU, zero outside the signal, scale, split to LDS
-  float ymax = 0.f;
+  float ym[TN];
 #pragma unroll
   for (int n = 0; n < TN; ++n) {
     const int t = y0 + wn * WN + n * 32 + l32;
     const bool in = t >= 0 && t < L;
+    ym[n] = 0.f;
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         const float u = in ? leaky(acc[m][n][r], a.slope) : 0.f;
         const float v = in ? leaky(acc[m][n][r + 1], a.slope) : 0.f;
-        if constexpr (!BF) ymax = max3_abs(ymax, u, v);
+        if constexpr (!BF) ym[n] = max3_abs(ym[n], u, v);
         acc[m][n][r] = u;
         acc[m][n][r + 1] = v;
       }
   }
-  float sy = 1.f;
+  float sy = kScaleX;
+  unsigned done = 0;  // the lane's column blocks whose outputs are stored already
   if constexpr (!BF) {
-    ymax = block_max(ymax);
-    if (__builtin_isinf(ymax)) {  // the largest finite one
-      float f = 0.f;
-#pragma unroll
-      for (int m = 0; m < TM; ++m)
-#pragma unroll
-        for (int n = 0; n < TN; ++n)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float v = fabsf(acc[m][n][r]);
-            f = v < __builtin_inff() ? fmaxf(f, v) : f;
-          }
-      ymax = block_max(f);
+    float top;
+    const unsigned has_nan = again1 && nan_bits() ? 1u : 0u;
+    unsigned f = block_or<NW>(range_bits(ym, sy, top) | has_nan, vote[1]);
+    if ((f & 3u) == 1u) {
+      top = block_max<NW>(top, wmax);
+      if (top > 0.f) {
+        sy = pow2_scale(top);
+        f = block_or<NW>(range_bits(ym, sy, top) | has_nan, vote[2]);
+      }
     }
-    sy = ymax == 0.f || (ymax >= kXMin && ymax <= kXMax) ? kScaleX : pow2_scale(ymax);
+    if (f & 1u) {
+      // the outputs whose own columns of the intermediate do not fit
+      unsigned* cm = reinterpret_cast<unsigned*>(sm);
+      for (int u = tid; u < YW; u += NT) cm[u] = 0u;
+      __syncthreads();
+#pragma unroll
+      for (int n = 0; n < TN; ++n) {
+        unsigned t = 0;
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) t = max(t, __builtin_bit_cast(unsigned, acc[m][n][r]) & 0x7fffffffu);
+        atomicMax(cm + wn * WN + n * 32 + l32, t);
+      }
+      __syncthreads();
+      done = unfit_bits(cm, 1, sy);
+#pragma unroll
+      for (int n = 0; n < TN; ++n)
+        if (wn * WN + n * 32 + l32 >= cols) done &= ~(1u << n);
+      if (block_or<NW>(done ? 1u : 0u, vote[0])) {
+        float* yf = reinterpret_cast<float*>(sm);  // [C][YS]
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int n = 0; n < TN; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              yf[(co_l + m * 32 + (r & 3) + 8 * (r >> 2)) * YS + wn * WN + n * 32 + l32] = acc[m][n][r];
+        for (int u = tid; u < C * (K - 1); u += NT) {
+          const int row = u / (K - 1);
+          yf[row * YS + BN + u - row * (K - 1)] = 0.f;
+        }
+        __syncthreads();
+        if (__any(done != 0u)) {
+          form_again(done, G.f2, G.b2, [&](float(&B)[TN], int k, int c) {
+#pragma unroll
+            for (int n = 0; n < TN; ++n) B[n] = yf[(c + half) * YS + wn * WN + n * 32 + l32 + k];
+          });
+          store(done);
+        }
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int n = 0; n < TN; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              acc[m][n][r] = yf[(co_l + m * 32 + (r & 3) + 8 * (r >> 2)) * YS + wn * WN + n * 32 + l32];
+      }
+      __syncthreads();  // the room is free again
+    }
   }
   first(uniform_rsrc(G.w2.w, wbytes));
   uint2* ys = reinterpret_cast<uint2*>(sm);  // [part][C / 8][YW][half]
@@ -320,8 +415,8 @@ void resblock_pair_kernel(PairLaunch a) {
                                          pk_bf16(acc[m][n][4 * q + 2], acc[m][n][4 * q + 3]));
         } else {
           uint2 h, l;
-          split2_inf(acc[m][n][4 * q] * sy, acc[m][n][4 * q + 1] * sy, h.x, l.x);
-          split2_inf(acc[m][n][4 * q + 2] * sy, acc[m][n][4 * q + 3] * sy, h.y, l.y);
+          split2(acc[m][n][4 * q] * sy, acc[m][n][4 * q + 1] * sy, h.x, l.x);
+          split2(acc[m][n][4 * q + 2] * sy, acc[m][n][4 * q + 3] * sy, h.y, l.y);
           ys[2 * at + half] = h;
           ys[2 * (at + (C / 8) * YW) + half] = l;
         }
@@ -339,12 +434,17 @@ void resblock_pair_kernel(PairLaunch a) {
 #pragma unroll 1
   for (int c = 0; c < nchunk; ++c)
     taps(w2, sm + (XU * c + half) * YW + wn * WN + l32, BF ? 2 * YW : (C / 8) * YW, 1);
-  const int cols = min(BO, L - o0);
-  const bool redo2 = !BF && any_nan(cols);
+  unsigned nan2 = 0;  // NaN sums of fitting columns: the weights'
+  if constexpr (!BF) {
+    nan2 = nan_bits() & ~done;
+#pragma unroll
+    for (int n = 0; n < TN; ++n)
+      if (wn * WN + n * 32 + l32 >= cols) nan2 &= ~(1u << n);
+  }
   finish(G.w2.sc, 1.f / sy, G.b2);
-  if (redo2) {
+  if (__any(nan2 != 0u)) {
     const float inv = 1.f / sy;
-    form_again(G.f2, G.b2, [&](float(&B)[TN], int k, int c) {
+    form_again(nan2, G.f2, G.b2, [&](float(&B)[TN], int k, int c) {
       const int ci = c + half;
 #pragma unroll
       for (int n = 0; n < TN; ++n) {
@@ -354,22 +454,7 @@ void resblock_pair_kernel(PairLaunch a) {
       }
     });
   }
-  const __amdgpu_buffer_rsrc_t rrs = uniform_rsrc(xb, 4u * (unsigned)(C * L));
-  const __amdgpu_buffer_rsrc_t ors = uniform_rsrc(G.out + (long long)b * C * L, 4u * (unsigned)(C * L));
-#pragma unroll
-  for (int m = 0; m < TM; ++m)
-#pragma unroll
-    for (int n = 0; n < TN; ++n) {
-      const int col = wn * WN + n * 32 + l32;
-      const unsigned oo = col < cols ? 4u * (unsigned)(co_l * L + o0 + col) : kBufOut;
-      float pre[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) pre[r] = buf_load4(rrs, oo, 4 * (m * 32 + (r & 3) + 8 * (r >> 2)) * L);
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[m][n][r] + pre[r]), ors, oo,
-                                              4 * (m * 32 + (r & 3) + 8 * (r >> 2)) * L, 0);
-    }
+  store(~done);
 }
 
 template <bool BF, int C, int BN, int WM, int WN>
@@ -379,13 +464,13 @@ void launch_p(PairLaunch a, hipStream_t s) {
   long long items = 0;
   for (int g = 0; g < a.n; ++g) {
     const int K = a.g[g].K;
-    units = std::max(units, (size_t)std::max(8 * (BN + (K - 1) * a.g[g].dil), (BF ? 1 : 2) * (C / 8) * (BN + K - 1)));
+    units = std::max(units, (size_t)std::max(8 * (BN + (K - 1) * a.g[g].dil), BF ? C / 8 * (BN + K - 1) : C / 4 * (BN + kConvTapsMax - 1)));
     a.g[g].tiles = (a.L + BN - K) / (BN - K + 1);
     items += (long long)a.g[g].tiles * a.B;
   }
   RVC_CHECK(items < (1LL << 30), "resblock_pair: launch too large");
   const size_t lds = units * sizeof(uint4);
-  constexpr size_t kMax = sizeof(uint4) * (size_t)std::max(8 * (BN + kConvHaloMax), (BF ? 1 : 2) * (C / 8) * (BN + kConvTapsMax - 1));
+  constexpr size_t kMax = sizeof(uint4) * (size_t)std::max(8 * (BN + kConvHaloMax), C / (BF ? 8 : 4) * (BN + kConvTapsMax - 1));
   static_assert(kMax <= 160 * 1024, "LDS of one workgroup");
   if constexpr (kMax > 65536) {
     static bool attr = false;  // per instantiation

@@ -102,14 +102,6 @@ __device__ __forceinline__ void split2(float a, float b, unsigned& h, unsigned& 
   h = __builtin_bit_cast(unsigned, hv);
   l = __builtin_bit_cast(unsigned, __builtin_convertvector(r, halfx2));
 }
-// the same with an infinity as (inf, 0)
-__device__ __forceinline__ void split2_inf(float a, float b, unsigned& h, unsigned& l) {
-  const halfx2 hv = __builtin_convertvector(floatx2{a, b}, halfx2);
-  const float ha = (float)hv.x, hb = (float)hv.y;
-  const floatx2 r = {a == ha ? 0.f : a - ha, b == hb ? 0.f : b - hb};
-  h = __builtin_bit_cast(unsigned, hv);
-  l = __builtin_bit_cast(unsigned, __builtin_convertvector(r, halfx2));
-}
 // the power of two that moves m (finite, above 0) into [2^14, 2^15), within the
 // normal floats on both sides of 1: what lies up to 2^14 below it is held too
 __device__ __forceinline__ float pow2_scale(float m) {

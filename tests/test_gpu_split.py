@@ -91,7 +91,7 @@ def test_infinity_reaches_what_it_reaches_in_fp32(decoders, name):
     assert np.isnan(got[np.isnan(want)]).all()
 
 
-@pytest.mark.parametrize("name", ["plain"])
+@pytest.mark.parametrize("name", sorted(GEOMS))
 @pytest.mark.parametrize("exponent", [24, 60, 100])
 def test_a_spike_takes_nothing_from_its_neighbours(decoders, name, exponent):
     """The samples that frames of huge or infinite z do not reach share tiles with
