@@ -69,14 +69,14 @@ __global__ __launch_bounds__(64 * NW) void conv2d_split_kernel(Conv2dLaunch a, i
 #pragma unroll
       for (int j = 0; j < 8; ++j) xv[e][j] = buf_load4(rs, xo[e], j * xrow);
   };
-  float sx = kScaleX, xmax = 0.f;
+  float sx = kScaleX, xm[2];  // each unit's largest magnitude, scaled
   auto lstore = [&]() __attribute__((always_inline)) {
     // a wave's LDS operations run in order; the fences keep the compiler to it
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int e = 0; e < 2; ++e)
-      if (lane + 64 * e < 2 * np) stage_unit<false>(xv[e], sx, xmax, xs + lane + 64 * e, 2 * np);
+      if (lane + 64 * e < 2 * np) stage_unit<false>(xv[e], sx, xm[e], xs + lane + 64 * e, 2 * np);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
@@ -91,9 +91,11 @@ __global__ __launch_bounds__(64 * NW) void conv2d_split_kernel(Conv2dLaunch a, i
   const uint4* xp = xs + half * np + (l32 >> tcs) * WC + (l32 & (TC - 1));
 
   floatx16 acc;
+  bool mixed = false;  // some units lie outside the split's range
   for (bool again = false;; again = true) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    xm[0] = xm[1] = 0.f;
     gload(c_lo);
     const unsigned last = (unsigned)(n * T - 1) * 2u * wpart;
     unsigned next = (unsigned)(c_lo * T) * 2u * wpart;
@@ -131,27 +133,48 @@ __global__ __launch_bounds__(64 * NW) void conv2d_split_kernel(Conv2dLaunch a, i
         Ah[1] = h; Al[1] = l;
       }
     }
-    if (again) break;
-    // the wave's largest magnitude: again with a scale of its own where fp16's
-    // range does not hold it
-    float m = xmax;
+    float top;
+    const unsigned f = range_bits(xm, 1.f, top);
+    mixed = __any(f & 1u);
+    if (!mixed || again || __any(f & 2u)) break;
+    // no unit fits: again with a scale of the wave's own
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
-    m = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m)));
-    if (m == 0.f || (m >= kXMin * kScaleX && m <= kXMax * kScaleX) || __builtin_isinf(m)) break;
-    sx = pow2_scale(m * (1.f / kScaleX));
+    for (int d = 32; d > 0; d >>= 1) top = fmaxf(top, __shfl_xor(top, d));
+    top = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, top)));
+    if (top == 0.f) break;  // infinities and zeros
+    sx = pow2_scale(top * (1.f / kScaleX));
   }
 
   const int pr = a0 + (l32 >> tcs), pc = b0 + (l32 & (TC - 1));
+  // the points whose own inputs the scale does not hold, or whose sums are NaN
+  bool bad = false;
+  if (mixed) {
+    unsigned* cm = reinterpret_cast<unsigned*>(xs);  // a position's largest magnitude, over the wave's window
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (lane < np) cm[lane] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int u = lane + 64 * e;
+      if (u < 2 * np) atomicMax(cm + (u < np ? u : u - np), __builtin_bit_cast(unsigned, xm[e]));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    unsigned t = 0;
+    for (int k = 0; k < T; ++k) t = max(t, cm[(l32 >> tcs) * WC + (l32 & (TC - 1)) + tap_off(k)]);
+    bad = !split_holds(__builtin_bit_cast(float, t));
+  }
   float nan = 0.f;
 #pragma unroll
   for (int r = 0; r < 16; ++r) nan = fmaf(acc[r], 0.f, nan);
-  const bool redo = __any(nan != nan);
+  bad = bad || nan != nan;
   const __amdgpu_buffer_rsrc_t srs = uniform_rsrc(G.wsc, 128u * (unsigned)n_row);
 #pragma unroll
   for (int r = 0; r < 16; ++r)
     acc[r] *= buf_load4(srs, 4u * (unsigned)(co0 + 4 * half), 4 * ((r & 3) + 8 * (r >> 2))) * (1.f / sx);
-  if (redo) {  // a NaN among the sums: this wave's channels again in fp32
+  if (__any(bad)) {  // this wave's channels again in fp32
     floatx16 f[1][1];
     const __amdgpu_buffer_rsrc_t frs = uniform_rsrc(G.w, 4u * (unsigned)(T * a.C_in * a.w_ld));
     const unsigned fo = co0 + l32 < a.C_out ? 4u * (unsigned)(half * a.w_ld + co0 + l32) : kBufOut;
@@ -166,7 +189,8 @@ __global__ __launch_bounds__(64 * NW) void conv2d_split_kernel(Conv2dLaunch a, i
           const int h = pr + G.dh[t], w = pc + G.dw[t];
           B[0] = buf_load4(rs, h >= 0 && h < a.H && w >= 0 && w < a.W ? half * xrow + 4u * (unsigned)(h * a.W + w) : kBufOut, 0);
         });
-    acc = f[0][0];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = bad ? f[0][0][r] : acc[r];
   }
 
   // ---- partial tiles [wave][channel][point], added in wave order

@@ -71,3 +71,37 @@ def test_infinities(weights):
     got, want = _hidden(inf, x), _hidden(low, x)
     assert np.isfinite(got).all()
     assert rel_l2(got, want) < 1e-6
+
+
+@pytest.mark.parametrize("exponent", [16, 24])
+def test_a_burst_takes_nothing_from_its_neighbours(weights, exponent):
+    """A burst in silence, with the image's scale such that the burst is about
+    2^20 times the silence, and the first encoder level cut down to one block:
+    the frames that the burst does not reach share tiles with those it does, and
+    are those of silence alone, within the error of two fp32 computations."""
+    silence, F = np.zeros(16000, np.float32), 101
+    burst = silence.copy()
+    burst[8000:8800] = 0.5 * np.random.default_rng(1).standard_normal(800, dtype=np.float32)
+    sd = dict(weights)
+    p = "unet.encoder.bn."
+    sd[p + "weight"] = np.full(1, 2.0 ** exponent, np.float32)
+    sd[p + "bias"] = np.full(1, 2.0 ** (exponent - 18), np.float32)
+    sd[p + "running_var"] = np.ones(1, np.float32)
+    sd[p + "running_mean"] = np.full(1, np.log(1e-5), np.float32)
+    for i in (1, 2, 3):
+        for k in ("weight", "bias"):
+            q = f"unet.encoder.layers.0.conv.{i}.conv.4.{k}"
+            sd[q] = np.zeros_like(sd[q])
+    m = HipRMVPE(sd)
+    level = []
+    for x in (silence, burst):
+        m.mel2hidden_from_audio(x)
+        level.append(m.read("cat0", (32, m.padded(F), 128))[16:])
+    m.close()
+    # the burst's samples lie in the windows of frames 47 .. 58, and each of the
+    # block's two 3x3 convolutions reaches one frame further (the padding behind
+    # frame 100 is as large as the burst)
+    off = np.abs(level[1] - level[0]).max(axis=(0, 2)) / np.abs(level[0][:, :90]).max()
+    assert (off[45:61] > 10).all()
+    for near in (slice(40, 45), slice(61, 66)):
+        assert rel_l2(level[1][:, near], level[0][:, near]) < 2e-6
