@@ -75,7 +75,7 @@ struct Synth : SessionBase {
     std::vector<float*> phases;
     float* up_b;
     float *nw, *nb;
-    float* rw[3][2][3];
+    float* rw[3][2][3];               // null at precision 2
     float* rb[3][2][3];
     std::vector<uint16_t*> phases16;  // precision >= 1
     uint16_t* rw16[3][2][3];          // precision 2, else null
@@ -448,7 +448,8 @@ struct Synth : SessionBase {
           for (int g = 0; g < 3; ++g) {
             const std::string rb = "dec.resblocks." + std::to_string(3 * i + j) + (l == 0 ? ".convs1." : ".convs2.") +
                                    std::to_string(g);
-            S.rw[j][l][g] = upload_conv(rb, c, c, ks[j], true);
+            // fp32 besides the two fp16 parts: for what those do not hold
+            S.rw[j][l][g] = precision >= 2 ? nullptr : upload_conv(rb, c, c, ks[j], true);
             S.rw16[j][l][g] = upload_conv16(precision >= 2, rb, c, c, ks[j], true);
             if (conv1d_split_supported(c, c, ks[j], 2 * g + 1, precision >= 2)) {
               const std::vector<float> hw = conv_host(rb, c, c, ks[j], true);

@@ -230,3 +230,27 @@ def test_config5_full_size_snr():
     assert min(snr1) >= 40.0
     assert min(snr2) >= 20.0
     assert np.isfinite(y2).all() and np.abs(y2).max() <= 1.0
+
+
+def test_bf16_resblocks_hold_no_fp32_weights():
+    """Beside the upsamplers' (bf16 in both), a session with bf16 ResBlocks holds
+    their weights in bf16 only: twice, in the layouts of its two kernels; one
+    with fp32 ResBlocks holds them in fp32 and in two fp16 parts."""
+    from rvc_hip import _hip
+    from rvc_hip.synth import HipSynthesizer
+
+    def free():
+        f, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert _hip.get_lib().hipMemGetInfo(ctypes.byref(f), ctypes.byref(total)) == 0
+        return f.value
+
+    w = syn.make_weights(syn.GEOM_40K, seed=0)
+    used = []
+    for precision in (0, 1, 2):  # the first one loads the code too
+        before = free()
+        s = HipSynthesizer(w, sr=syn.GEOM_40K.sr, precision=precision)
+        used.append(before - free())
+        s.close()
+    weights = 4 * sum(a.size for k, a in w.items() if k.startswith("dec.resblocks.") and k.endswith("weight_v"))
+    # half of the fp32 session's bytes, but for the allocator's granularity
+    assert used[1] - used[2] > 0.8 * weights
