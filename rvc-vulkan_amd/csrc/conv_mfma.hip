@@ -412,10 +412,6 @@ __device__ __forceinline__ void persist_tile(int lin, int n_tx, int n_ty, int& t
   }
 }
 
-// FAM only names the instantiation (1: the three-group stored launches of
-// the decoder ResBlocks), so profiles can tell them from the other launches
-// of the same tile; the code is identical.
-//
 // DIRECT (launches whose input takes no activation): chunks are staged by
 // direct-to-LDS buffer loads (lane i of a wave writes 4 or 16 bytes at the
 // wave's LDS base + 4i or 16i; out-of-range lanes write 0), so the staged
@@ -430,7 +426,7 @@ __device__ __forceinline__ void persist_tile(int lin, int n_tx, int n_ty, int& t
 // one base per tap, and the staging offsets need no division by a runtime
 // width.  HC = 0: the stride is the item's own window, BN + (K - 1) dil
 // (fewer registers: the 32-row tiles, which measured faster this way).
-template <int BM, int BN, int WM, int WN, int BK, int FAM, bool DIRECT = false, int HC = 0>
+template <int BM, int BN, int WM, int WN, int BK, bool DIRECT = false, int HC = 0>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64)
 __attribute__((amdgpu_waves_per_eu(4)))
 void conv1d_mfma_persist_kernel(ConvLaunch a, int n_tx, int n_ty, int stage_floats, int cpx) {
@@ -1728,33 +1724,27 @@ bool persist_ok(const ConvLaunch& a) {
 }
 
 template <int BM, int BN, int WM, int WN, int BK, bool DIRECT, int HC>
-bool launch_persist_kernel(const ConvLaunch& a, hipStream_t s, int stage, size_t lds, int n_tx, int n_ty, bool fam,
+bool launch_persist_kernel(const ConvLaunch& a, hipStream_t s, int stage, size_t lds, int n_tx, int n_ty,
                            long long items) {
   using C = Cfg<BM, BN, WM, WN, BK, 1, 1, kConvTapsMax, 2>;
-  const void* k1 = reinterpret_cast<const void*>(&conv1d_mfma_persist_kernel<BM, BN, WM, WN, BK, 1, DIRECT, HC>);
-  const void* k0 = reinterpret_cast<const void*>(&conv1d_mfma_persist_kernel<BM, BN, WM, WN, BK, 0, DIRECT, HC>);
+  const void* kern = reinterpret_cast<const void*>(&conv1d_mfma_persist_kernel<BM, BN, WM, WN, BK, DIRECT, HC>);
   // 64 KiB of staging plus the kernel's static ticket word: allow the
   // dynamic part its full size (a CU holds 160 KiB)
   if (lds > 65536 - 256) {
     static bool attr = false;  // per instantiation
     if (!attr) {
-      RVC_HIP(hipFuncSetAttribute(k1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit));
-      RVC_HIP(hipFuncSetAttribute(k0, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit));
+      RVC_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit));
       attr = true;
     }
   }
-  const int per_cu = resident_blocks(fam ? k1 : k0, C::NT, lds);
+  const int per_cu = resident_blocks(kern, C::NT, lds);
   if (per_cu < 1) return false;
   long long grid = (long long)per_cu * device_cus();
   if (grid >= 8) grid -= grid % 8;  // item j then runs on XCD j % 8
   grid = std::min(grid, items);
   const int cpx = device_cus() % 8 == 0 ? device_cus() / 8 : 0;  // CUs per XCD
-  if (fam)
-    launch_timed(conv1d_mfma_persist_kernel<BM, BN, WM, WN, BK, 1, DIRECT, HC>, dim3((unsigned)grid), dim3(C::NT), lds,
-                 s, a, n_tx, n_ty, stage, cpx);
-  else
-    launch_timed(conv1d_mfma_persist_kernel<BM, BN, WM, WN, BK, 0, DIRECT, HC>, dim3((unsigned)grid), dim3(C::NT), lds,
-                 s, a, n_tx, n_ty, stage, cpx);
+  launch_timed(conv1d_mfma_persist_kernel<BM, BN, WM, WN, BK, DIRECT, HC>, dim3((unsigned)grid), dim3(C::NT), lds, s,
+               a, n_tx, n_ty, stage, cpx);
   check_launch("conv1d_mfma_persist");
   return true;
 }
@@ -1789,19 +1779,17 @@ bool launch_persist(const ConvLaunch& a, hipStream_t s) {
   const int n_ty = (a.C_out + BM - 1) / BM;
   const long long items = (long long)a.B * n_tx * n_ty * a.n_groups;
   RVC_CHECK(items < (1LL << 30), "conv1d_mfma: launch too large");
-  bool fam = a.n_groups == 3;
-  for (int g = 0; g < a.n_groups; ++g) fam = fam && a.g[g].combine == COMB_STORE;
   if constexpr (BM < 64) {
-    return direct ? launch_persist_kernel<BM, BN, WM, WN, BK, true, 0>(a, s, stage, lds, n_tx, n_ty, fam, items)
-                  : launch_persist_kernel<BM, BN, WM, WN, BK, false, 0>(a, s, stage, lds, n_tx, n_ty, fam, items);
+    return direct ? launch_persist_kernel<BM, BN, WM, WN, BK, true, 0>(a, s, stage, lds, n_tx, n_ty, items)
+                  : launch_persist_kernel<BM, BN, WM, WN, BK, false, 0>(a, s, stage, lds, n_tx, n_ty, items);
   } else {
     if (direct)
-      return HC == 16 ? launch_persist_kernel<BM, BN, WM, WN, BK, true, 16>(a, s, stage, lds, n_tx, n_ty, fam, items)
+      return HC == 16 ? launch_persist_kernel<BM, BN, WM, WN, BK, true, 16>(a, s, stage, lds, n_tx, n_ty, items)
                       : launch_persist_kernel<BM, BN, WM, WN, BK, true, kConvHaloMax>(a, s, stage, lds, n_tx, n_ty,
-                                                                                     fam, items);
-    return HC == 16 ? launch_persist_kernel<BM, BN, WM, WN, BK, false, 16>(a, s, stage, lds, n_tx, n_ty, fam, items)
+                                                                                     items);
+    return HC == 16 ? launch_persist_kernel<BM, BN, WM, WN, BK, false, 16>(a, s, stage, lds, n_tx, n_ty, items)
                     : launch_persist_kernel<BM, BN, WM, WN, BK, false, kConvHaloMax>(a, s, stage, lds, n_tx, n_ty,
-                                                                                    fam, items);
+                                                                                    items);
   }
 }
 

@@ -94,8 +94,8 @@ def is_resblock(kernel: str, grid) -> bool:
     if kernel.startswith("conv1d_split_kernel"):  # the last template argument is the stride: HuBERT's are 2
         return kernel[kernel.find("<") + 1:kernel.rfind(">")].replace(" ", "").split(",")[-1] == "1"
     if kernel.startswith("conv1d_mfma_persist_kernel"):
-        # template arguments <BM, BN, WM, WN, BK, FAM[, DIRECT]>: FAM = 1 marks
-        # the three-group stored launches
+        # traces of the ResBlocks on the fp32 matrix cores: template arguments
+        # <BM, BN, WM, WN, BK, FAM[, DIRECT]>, FAM = 1 for the three-group stored launches
         args = kernel[kernel.find("<") + 1:kernel.rfind(">")].replace(" ", "").split(",")
         return len(args) >= 6 and args[5] == "1"
     return kernel.startswith("conv1d_mfma_kernel") and grid[2] == 3 and grid[0] >= 64
