@@ -28,8 +28,13 @@
 // them, or a NaN among the sums) are formed on the fp32 matrix cores from the
 // fp32 weights (fp32_sums), which gives what an fp32 convolution gives.  So an
 // output has fp32's precision and reach whatever else is in its tile, as far
-// as its inputs go; within an output's own inputs, channels or taps far below
-// the largest keep 2^-31 absolute (2^-40 of the row's largest weight).
+// as its inputs go.  Within an output's own inputs, channels or taps far below
+// the largest keep 2^-31 absolute, and weights 2^-34 of their row's largest:
+// where small inputs meet large weights and large inputs small ones, the error
+// is the fp32 matrix cores' up to a spread of 2^10 between channels and
+// grows with it from there (a ResBlock whose intermediate channels spread over
+// 2^10 / 2^14 / 2^18, the next conv's weights making up for it: 2.2e-7 / 1.4e-6
+// / 1.9e-5, fp32 2.1e-7).
 //
 // One workgroup forms a BM x BN tile, wave (wm, wn) a WM x WN part of it, over
 // chunks of 16 input channels.  A chunk's input window (BN + (K - 1) dil
