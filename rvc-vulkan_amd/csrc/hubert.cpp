@@ -321,15 +321,16 @@ struct Hubert : SessionBase {
     float* part = buf("attn_part", part_n);
     const int nl = version == 1 ? 9 : n_layers;
     // Post-LN layers: x1 = LN1(x + o-proj(attn)), x' = LN2(x1 + FFN(x1)).
-    // When the four 1x1 GEMMs of a layer run on the chunked small-conv
-    // kernel (L up to about 950 frames), neither LayerNorm is a launch of its
+    // When the four 1x1 GEMMs of a layer run on split products (widths above 256
+    // that are multiples of 64, any length) or on the chunked small-conv
+    // kernel (multiples of 128, few tiles), neither LayerNorm is a launch of its
     // own and no normalised tensor is stored: the o-projection and the FFN
     // output GEMM also write the column statistics of their 32-row tiles
-    // (st1, st2), the FFN input / next q/k/v GEMM normalise their input while
-    // staging it, and the GEMM that adds the normalised tensor as its
+    // (st1, st2), the FFN input / next q/k/v GEMM normalise their input on the
+    // way in, and the GEMM that adds the normalised tensor as its
     // residual normalises the raw one in its epilogue.  Only the last
-    // layer's LN2 is a LayerNorm launch.  Longer inputs (split-K GEMMs) keep
-    // the LayerNorm launches.
+    // layer's LN2 is a LayerNorm launch.  Other widths keep the LayerNorm
+    // launches.
     const int nt = H / 32;
     double* st1 = reinterpret_cast<double*>(buf("ln_stat1", (size_t)4 * B * nt * L));
     double* st2 = reinterpret_cast<double*>(buf("ln_stat2", (size_t)4 * B * nt * L));

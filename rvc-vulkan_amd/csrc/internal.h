@@ -163,7 +163,7 @@ struct ConvGroup {
   int combine;
   const uint16_t* w16;  // bf16 launches: weights [K][C_out][w16_ld] in bf16, 16-byte aligned
   int tiles;          // output tiles per workgroup (set by the launcher)
-  const uint16_t* wsp;  // split launches: weights in two fp16 parts (SessionBase::pack_split), 16-byte aligned
+  const uint16_t* wsp;  // split launches: weights in two fp16 parts (SessionBase::upload_split), 16-byte aligned
   const float* wsc;     // and each output row's scale: weight = (h + l) * wsc[row]
 };
 

@@ -53,9 +53,6 @@ __device__ __forceinline__ void topk_insert(float (&bs)[kTopK], int (&bi)[kTopK]
   }
 }
 
-// Partial top-k of one slice of database rows for 64 queries (one per lane):
-// dist = (q2[f] + d2[n]) - 2 * dot[n][f], clamped at 0
-// (runtime/retrieval.py:56-62).  Writes [slice][F][kTopK].
 // Index rows in two fp16 parts and a scale each, in the operand order of
 // SessionBase::upload_split (one tap); rows from N on are zero.  A workgroup takes
 // 32 rows (a row block), 8 lanes a row; once per index, bound by its writes.
@@ -89,6 +86,9 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* v, int N, 
   }
 }
 
+// Partial top-k of one slice of database rows for 64 queries (one per lane):
+// dist = (q2[f] + d2[n]) - 2 * dot[n][f], clamped at 0
+// (runtime/retrieval.py:56-62).  Writes [slice][F][kTopK].
 __global__ __launch_bounds__(64) void knn_partial_kernel(const float* dot, long long ldd, const float* q2,
                                                          const float* d2, int F, int N, int per, float* ps, int* pi) {
 #pragma clang fp contract(off)

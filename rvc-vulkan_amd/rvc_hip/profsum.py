@@ -101,6 +101,12 @@ def is_resblock(kernel: str, grid) -> bool:
     return kernel.startswith("conv1d_mfma_kernel") and grid[2] == 3 and grid[0] >= 64
 
 
+def resblock_convs(kernel: str) -> int:
+    """Grouped convolutions one ResBlock dispatch stands for: a fused pair is two,
+    as the session's timing counts it."""
+    return 2 if kernel.startswith("resblock_pair_kernel") else 1
+
+
 def _counter_means(db: str, counter: str):
     """{(kernel, grid): (mean KiB per dispatch, dispatches)} for one counter."""
     return {(r["kernel"], r["grid"]): (r["mean"], r["n"]) for r in pmc_rows(db) if r["counter"] == counter}
@@ -133,9 +139,9 @@ def traffic(fetch_db: str, write_db: str, copy_fetch: str, copy_write: str, mib:
         print(f"| {k[0]} | {k[1]} | {n} | {rd / 1e6:.2f} | {wr / 1e6:.2f} | {(rd + wr) / 1e6:.2f} |")
         if is_resblock(*k):
             fam_b += (rd + wr) * n
-            fam_n += n
+            fam_n += n * resblock_convs(k[0])
     if fam_n:
-        print(f"\nResBlock family (persistent FAM 1, or one-shot grid z = 3 and >= 64 wide): {fam_n} dispatches")
+        print(f"\nResBlock family (resblock_pair and conv1d_split, a pair counted as its two convolutions): {fam_n} launches")
         print(f"resblock_traffic_bytes_per_launch: {int(round(fam_b / fam_n))}")
     return 0
 
@@ -198,7 +204,7 @@ def sq_summary(db_a: str, db_b: str = None) -> int:
             fam[1] += N_SIMD * d * PEAK_GHZ * 1e9 * n[k]
             fam[2] += N_SIMD * d * clk * 1e9 * n[k]
     if fam[1] > 0:
-        print(f"\nResBlock family (persistent FAM 1, or one-shot grid z = 3 and >= 64 wide):")
+        print("\nResBlock family (resblock_pair and conv1d_split):")
         print(f"resblock_mfma_busy_at_peak_clock: {fam[0] / fam[1]:.3f}")
         print(f"resblock_mfma_busy_at_run_clock: {fam[0] / fam[2]:.3f}")
     return 0
@@ -239,7 +245,7 @@ def main(argv=None):
     n = sum(r["calls"] for r in rb)
     tot = sum(r["total_ms"] for r in rb)
     if n:
-        print(f"\nResBlock family (persistent FAM 1, or one-shot grid z = 3 and >= 64 wide): {n} dispatches, "
+        print(f"\nResBlock family (resblock_pair and conv1d_split): {n} dispatches, "
               f"{tot:.2f} ms total, average {tot * 1e3 / n:.1f} us per dispatch")
     allk = sum(r["total_ms"] for r in rows)
     print(f"all kernels: {allk:.2f} ms" + (f", {allk / args.steps:.3f} ms per step" if args.steps else ""))

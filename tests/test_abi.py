@@ -217,3 +217,16 @@ def test_profile_summary_resblock_family():
     assert not is_resblock("conv1d_mfma_persist_kernel<64, 256, 32, 64, 8, 0, true>", (512, 1, 1))
     assert is_resblock("conv1d_mfma_kernel<64, 128, 32, 64, 8, 1, 1, 11, 1>", (79, 2, 3))
     assert not is_resblock("conv1d_mfma_kernel<64, 128, 32, 64, 8, 1, 1, 11, 1>", (79, 2, 1))
+
+
+def test_profile_summary_split_resblocks():
+    """The split kernels in the ResBlock family: HuBERT's stride-2 convs are not
+    (the last template argument), and a fused pair stands for two launches."""
+    from rvc_hip.profsum import is_resblock, resblock_convs
+
+    pair = "resblock_pair_kernel<false, 128, 128, 32, 128>"
+    conv = "conv1d_split_kernel<false, 64, 128, 32, 64, 1>"
+    assert is_resblock(pair, (2462, 1, 1)) and is_resblock(conv, (948, 1, 1))
+    assert not is_resblock("conv1d_split_kernel<false, 64, 128, 32, 64, 2>", (948, 1, 1))
+    assert not is_resblock("conv1d_mfma_persist_kernel<64, 256, 32, 64, 8, true, 16>", (512, 1, 1))
+    assert (resblock_convs(pair), resblock_convs(conv)) == (2, 1)

@@ -107,10 +107,10 @@ def test_long_input_feature_extractor_vs_oracle(sd, hub):
 
 
 def test_long_input_layernorm_launches_vs_oracle(sd, hub):
-    """20 s of input (999 frames): the FFN input GEMM's tiles leave the
-    chunked small-conv kernel, so every LayerNorm runs as a launch of its own
-    instead of inside the neighbouring GEMMs (the path of shorter inputs,
-    which the tests above cover); the output against the oracle's."""
+    """20 s of input (999 frames), a length at which the fp32 GEMMs took
+    LayerNorm launches; at this width the split GEMMs carry the LayerNorms
+    at every length (test_gpu_hubert_split.py covers the launches); the output
+    against the oracle's."""
     x = syn.make_hubert_input(320000, seed=10)
     got = hub.encode(x, version=2)
     want = H.HubertRef(sd).encode(x, version=2)
