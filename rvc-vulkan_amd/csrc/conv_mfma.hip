@@ -1299,33 +1299,14 @@ __global__ __launch_bounds__(64 * NW) void conv_small_kernel(ConvLaunch a) {
   const float* wl = ws + (wave * Q + half) * 32 + l32;
   const float* xl = xs + (wave * Q + half) * XW + l32;
   load(c_lo);
-  // LayerNorms from the producers' column statistics (1x1 launches only;
-  // a thread stages and finishes one column, tid % BN): of the input while
-  // it is staged (no affine: the caller folds gamma / beta into the weights
-  // and bias), and of the residual in the epilogue.  xs is free until the
-  // first chunk is staged and holds the statistics' scratch.
-  constexpr bool kLn = K == 1;
-  static_assert(!kLn || (NT % BN == 0 && XE * NT >= 4 * NT + 2 * BN), "a thread stages one column; scratch room");
-  const bool ln = kLn && a.ln_stat != nullptr;
-  float ln_mu = 0.f, ln_rd = 0.f, rs_mu = 0.f, rs_rd = 0.f;
-  if constexpr (kLn) {
-    if (ln) ln_column_stats<NT, BN>(a.ln_stat, a.ln_ntile, C_in, a.L_in, a.ln_eps, b, i0, xs, ln_mu, ln_rd);
-    if (a.res_stat && nsplit == 1)
-      ln_column_stats<NT, BN>(a.res_stat, a.C_out / 32, a.C_out, G.n_out, a.ln_eps, b, i0, xs, rs_mu, rs_rd);
-  }
   for (int c = c_lo; c < c_hi; ++c) {
 #pragma unroll
     for (int j = 0; j < WF4; ++j) reinterpret_cast<float4*>(ws)[j * NT + tid] = wv[j];
-    if (ln) {
 #pragma unroll
-      for (int j = 0; j < XE; ++j) xs[j * NT + tid] = (xv[j] - ln_mu) * ln_rd;
-    } else {
-#pragma unroll
-      for (int j = 0; j < XE; ++j) {
-        float u = xv[j];
-        if (leaky) u = u >= 0.f ? u : u * a.in_slope;
-        xs[j * NT + tid] = u;
-      }
+    for (int j = 0; j < XE; ++j) {
+      float u = xv[j];
+      if (leaky) u = u >= 0.f ? u : u * a.in_slope;
+      xs[j * NT + tid] = u;
     }
     __syncthreads();
     if (c + 1 < c_hi) load(c + 1);
@@ -1345,7 +1326,7 @@ __global__ __launch_bounds__(64 * NW) void conv_small_kernel(ConvLaunch a) {
     }
     if (c + 1 < c_hi) __syncthreads();  // the next chunk's stores overwrite this one
   }
-  small_conv_epilogue<BN, NW>(a, G, b, i0, co0, gate, acc, smem, rs_mu, rs_rd, nsplit > 1 ? sidx : -1);
+  small_conv_epilogue<BN, NW>(a, G, b, i0, co0, gate, acc, smem, 0.f, 0.f, nsplit > 1 ? sidx : -1);
 }
 
 // 1x1 convolutions with long reductions (HuBERT's linear layers: C_in 512 ..
@@ -1491,13 +1472,10 @@ void conv1x1_split_kernel(ConvLaunch a, int n_row, int n_col) {
 
 // The output of a split chunked 1x1 launch (sc_split > 1): for output column
 // i of 32-row tile blockIdx.y, out = ((sum_s part[s]) + bias) + res, the
-// splits added in index order and the residual normalised from a.res_stat
-// when set (the small-conv epilogue's formulas); with a.stat_out, the float64
-// (sum, sum of squares) of the tile's stored values per column.  A workgroup
+// splits added in index order.  A workgroup
 // takes kSrCols columns x the tile's 32 rows, thread (g, c) rows kSrRows * g
-// .. + kSrRows - 1 of column c, every operand loaded before the first store;
-// the statistics are added per thread in row order, then over g in order.
-constexpr int kSrCols = 32, kSrRows = 4, kSrGroups = 256 / kSrCols;  // 384 workgroups at 499 frames
+// .. + kSrRows - 1 of column c, every operand loaded before the first store.
+constexpr int kSrCols = 32, kSrRows = 4, kSrGroups = 256 / kSrCols;  // 384 workgroups at 768 rows, 499 columns
 static_assert(kSrGroups * kSrRows == 32, "a workgroup covers the 32 rows of its tile");
 __global__ __launch_bounds__(256) void splitk_small_reduce_kernel(ConvLaunch a) {
   const ConvGroup& G = a.g[0];
@@ -1505,21 +1483,7 @@ __global__ __launch_bounds__(256) void splitk_small_reduce_kernel(ConvLaunch a) 
   const int i = blockIdx.x * kSrCols + c;
   const int tile = blockIdx.y, b = blockIdx.z;
   const bool icol = i < G.n_out;
-  const int S = a.sc_split, ntile = a.C_out / 32;
-  __shared__ double red[kSrGroups][kSrCols][2];
-  float mu = 0.f, rd = 0.f;
-  if (a.res_stat && icol) {
-    const double2* st = reinterpret_cast<const double2*>(a.res_stat) + (long long)b * ntile * G.n_out + i;
-    double sm = 0.0, sq = 0.0;
-    for (int t = 0; t < ntile; ++t) {
-      const double2 w = st[(long long)t * G.n_out];
-      sm += w.x;
-      sq += w.y;
-    }
-    const double md = sm / a.C_out;
-    mu = (float)md;
-    rd = 1.0f / sqrtf((float)(fmax(sq - sm * md, 0.0) / a.C_out) + a.ln_eps);
-  }
+  const int S = a.sc_split;
   constexpr unsigned kOut = 0x80000000u;
   const int r0 = tile * 32 + kSrRows * rg;  // this thread's first row
   const unsigned plane = 4u * (unsigned)(a.B * a.C_out * G.n_out);  // bytes of one split's partials
@@ -1541,35 +1505,14 @@ __global__ __launch_bounds__(256) void splitk_small_reduce_kernel(ConvLaunch a) 
     for (int r = 0; r < kSrRows; ++r)
       v[r] = v[r] + __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(prs, pu, 4 * r * G.n_out, 0));
   }
-  double sm = 0.0, sq = 0.0;
-  if (icol) {
-    float* op = G.out + (long long)b * a.ob + (long long)r0 * a.oc + i;
+  if (!icol) return;
+  float* op = G.out + (long long)b * a.ob + (long long)r0 * a.oc + i;
 #pragma unroll
-    for (int r = 0; r < kSrRows; ++r) {
-      const int co = r0 + r;
-      float t = v[r];
-      if (G.bias) t = t + G.bias[co];
-      if (hr) {
-        float x = rv[r];
-        if (a.res_stat) x = (x - mu) * rd * a.res_g[co] + a.res_b[co];
-        t = t + x;
-      }
-      op[(long long)r * a.oc] = t;
-      sm += t;
-      sq += (double)t * t;
-    }
-  }
-  if (!a.stat_out) return;  // uniform: no barrier follows
-  red[rg][c][0] = sm;
-  red[rg][c][1] = sq;
-  __syncthreads();
-  if (rg == 0 && icol) {
-    double tsm = red[0][c][0], tsq = red[0][c][1];
-    for (int g = 1; g < kSrGroups; ++g) {
-      tsm += red[g][c][0];
-      tsq += red[g][c][1];
-    }
-    reinterpret_cast<double2*>(a.stat_out)[((long long)b * ntile + tile) * G.n_out + i] = make_double2(tsm, tsq);
+  for (int r = 0; r < kSrRows; ++r) {
+    float t = v[r];
+    if (G.bias) t = t + G.bias[r0 + r];
+    if (hr) t = t + rv[r];
+    op[(long long)r * a.oc] = t;
   }
 }
 
@@ -1876,12 +1819,11 @@ bool small_conv_ok(const ConvLaunch& a) {
 // chunks at 499 frames) run as two splits (768 workgroups of 12 chunks, three
 // per CU), their raw partial tiles through part, and
 // splitk_small_reduce_kernel forms the output.  Plain epilogues only: bias,
-// a residual (LayerNorm'ed from statistics or not), column statistics out.
+// a residual.
 int small_conv_split(const ConvLaunch& a) {
   if (conv1x1_split_ok(a)) return 1;
   if (a.n_groups != 1 || a.g[0].K != 1 || a.C_in < 3072 || a.C_in % 256 != 0 || a.C_out % 32 != 0) return 1;
-  if (a.post != POST_NONE || a.out_act != ACT_NONE || a.in_act != ACT_NONE || a.bias2 || a.ln_stat || a.ln_g)
-    return 1;
+  if (a.post != POST_NONE || a.out_act != ACT_NONE || a.in_act != ACT_NONE || a.bias2 || a.ln_g) return 1;
   if (a.g[0].combine != COMB_STORE || a.g[0].in_step > 1 || small_gemm_ok(a) || !small_conv_ok(a)) return 1;
   return 2;
 }
@@ -1893,8 +1835,6 @@ void launch_small_conv_cfg(const ConvLaunch& a, dim3 grid, hipStream_t s) {
   constexpr size_t lds_stage = sizeof(float) * ((size_t)K * CHK * 32 + (size_t)XE * NT);
   constexpr size_t lds_red = sizeof(float) * NW * (BN / 32) * 16 * 64;  // the epilogue's partial tiles
   static_assert((lds_stage > lds_red ? lds_stage : lds_red) <= 160 * 1024, "staging LDS above the CU's 160 KiB");
-  RVC_CHECK((!a.ln_stat || a.ln_ntile <= 4 * (NT / BN)) && (!a.res_stat || a.C_out / 32 <= 4 * (NT / BN)),
-            "conv_small: too many statistics tiles for a staged LayerNorm");
   constexpr size_t lds = lds_stage > lds_red ? lds_stage : lds_red;
   // the gate epilogue pairs tile rows k and k + KO / 2 of one thread
   RVC_CHECK(a.post != POST_WN_GATE || 32 * BN / (64 * NW) >= 2,
@@ -2096,11 +2036,6 @@ bool conv1d_mfma_supported(int K, int dil) {
   return K >= 0 && K <= kConvTapsMax && dil >= 1 && (K > 0 ? (K - 1) * dil : 0) <= kConvHaloMax;
 }
 
-bool conv1d_mfma_chunked_1x1(const ConvLaunch& a) {
-  return conv1x1_split_ok(a) || (a.n_groups == 1 && a.g[0].K == 1 && (a.g[0].in_step <= 1) && a.post == POST_NONE &&
-                                 !small_gemm_ok(a) && small_conv_ok(a));
-}
-
 void launch_conv1d_mfma(const ConvLaunch& a, hipStream_t s) {
   RVC_CHECK(a.n_groups >= 1 && a.n_groups <= kMaxConvGroups, "conv1d_mfma: bad group count");
   RVC_CHECK(a.C_in >= 1 && a.C_out >= 1 && a.B >= 1 && a.w_ld >= a.C_out && a.w_ld % 4 == 0,
@@ -2116,20 +2051,16 @@ void launch_conv1d_mfma(const ConvLaunch& a, hipStream_t s) {
     RVC_CHECK((reinterpret_cast<uintptr_t>(a.g[g].w) & 15) == 0, "conv1d_mfma: weights must be 16-byte aligned");
   }
   if (max_n_out(a) == 0) return;
-  if (a.ln_stat) {
-    RVC_CHECK(conv1d_mfma_chunked_1x1(a) && a.in_act == ACT_NONE && a.ln_ntile >= 1 && a.ln_ntile * 32 == a.C_in,
-              "conv1d_mfma: a LayerNorm from producer statistics needs the chunked 1x1 kernel (one group, no input "
-              "activation, C_in / 32 statistics tiles)");
-  } else {
-    RVC_CHECK(!a.ln_g || (step == 1 && small_gemm_ok(a)),
-              "conv1d_mfma: a staged LayerNorm needs the whole-reduction 1x1 kernel (C_in <= 256, <= 8192 columns)");
-  }
-  RVC_CHECK(!a.stat_out || (step == 1 && a.n_groups == 1 && a.C_out % 32 == 0 && a.post == POST_NONE &&
-                            (conv1x1_split_ok(a) || small_gemm_ok(a) || small_conv_ok(a))),
-            "conv1d_mfma: column statistics need a small-conv kernel (one group, C_out % 32 == 0)");
-  RVC_CHECK(!a.res_stat || (conv1d_mfma_chunked_1x1(a) && a.C_out % 32 == 0 && a.g[0].res && a.res_g && a.res_b),
-            "conv1d_mfma: a residual LayerNorm needs the chunked 1x1 kernel, a residual, gamma and beta");
-  if (conv1x1_split_ok(a) && conv1x1_split_launch(a, s)) return;
+  const bool split1 = conv1x1_split_ok(a);
+  RVC_CHECK(!a.ln_g || (step == 1 && small_gemm_ok(a)),
+            "conv1d_mfma: a staged LayerNorm needs the whole-reduction 1x1 kernel (C_in <= 256, <= 8192 columns)");
+  RVC_CHECK((!a.ln_stat && !a.stat_out && !a.res_stat) || split1,
+            "conv1d_mfma: column statistics need the 1x1 kernel on split products");
+  RVC_CHECK(!a.ln_stat || (a.ln_ntile >= 1 && a.ln_ntile * 32 == a.C_in),
+            "conv1d_mfma: a LayerNorm from producer statistics takes C_in / 32 statistics tiles");
+  RVC_CHECK(!a.res_stat || (a.g[0].res && a.res_g && a.res_b),
+            "conv1d_mfma: a residual LayerNorm needs a residual, gamma and beta");
+  if (split1 && conv1x1_split_launch(a, s)) return;
   if (step == 1 && small_gemm_ok(a) && launch_small_gemm(a, s)) return;
   if (step == 1 && small_conv_ok(a) && launch_small_conv(a, s)) return;
   for (int g = 0; g < a.n_groups; ++g)

@@ -322,9 +322,8 @@ struct Hubert : SessionBase {
     const int nl = version == 1 ? 9 : n_layers;
     // Post-LN layers: x1 = LN1(x + o-proj(attn)), x' = LN2(x1 + FFN(x1)).
     // When the four 1x1 GEMMs of a layer run on split products (widths above 256
-    // that are multiples of 64, any length) or on the chunked small-conv
-    // kernel (multiples of 128, few tiles), neither LayerNorm is a launch of its
-    // own and no normalised tensor is stored: the o-projection and the FFN
+    // that are multiples of 64, at any length), neither LayerNorm is a launch of
+    // its own and no normalised tensor is stored: the o-projection and the FFN
     // output GEMM also write the column statistics of their 32-row tiles
     // (st1, st2), the FFN input / next q/k/v GEMM normalise their input on the
     // way in, and the GEMM that adds the normalised tensor as its
@@ -342,7 +341,7 @@ struct Hubert : SessionBase {
                                    with_split(c1x1(t1, HL, layers[0].wi, layers[0].bi, ff, B, H, F, (int)L), layers[0].si),
                                    with_split(c1x1(ff, (long long)F * L, layers[0].wf, layers[0].bf, t2, B, F, H, (int)L),
                                               layers[0].sf)};
-      for (const ConvLaunch& p : probe) fold = fold && conv1d_mfma_chunked_1x1(p);
+      for (const ConvLaunch& p : probe) fold = fold && conv1x1_split_ok(p);
     }
     auto ln_in = [&](ConvLaunch& c, const double* st) {  // the affine is in the folded weights
       c.ln_stat = st;

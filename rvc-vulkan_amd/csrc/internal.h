@@ -218,15 +218,15 @@ struct ConvLaunch {
   float* ln_out;
   long long ln_ob, ln_oc;
   float ln_eps;
-  // The same LayerNorm in the chunked small-conv kernel (1x1, single group),
-  // whose chunks cannot hold a whole column: the statistics come from the
+  // The same LayerNorm in the 1x1 kernel on split products (conv1x1_split_ok),
+  // whose waves do not hold a whole column: the statistics come from the
   // kernel that produced the input.  stat_out (producer, single group,
   // C_out % 32 == 0): per batch item, 32-row C_out tile and output column,
   // the float64 sum and sum of squares of the 32 values it stored, added in
   // row order, as double2 [B][C_out / 32][n_out].  ln_stat (consumer): its
   // input's statistics in that layout, ln_ntile = C_in / 32 tiles of L_in
-  // columns, added in tile order: mean = S / C_in, var = (Q - S * mean) /
-  // C_in, and x' = (x - mean) * (1 / sqrt(var + ln_eps)) while staging --
+  // columns, added in a fixed order: mean = S / C_in, var = (Q - S * mean) /
+  // C_in, and x' = (x - mean) * (1 / sqrt(var + ln_eps)) on the way in --
   // without the affine, which the caller folds into the weights (W diag(g))
   // and the bias (+ W b); ln_g / ln_b / ln_out unused.  res_stat: the
   // residual is such a raw tensor too (C_out channels, C_out / 32 tiles,
@@ -246,11 +246,9 @@ enum Post : int { POST_NONE = 0, POST_WN_GATE = 1, POST_WN_UPDATE = 2 };
 // MFMA implicit-GEMM conv1d (input stride 1 or 2, the same for every group
 // of a launch), K <= kConvTapsMax and (K-1)*dil <= kConvHaloMax.
 bool conv1d_mfma_supported(int K, int dil);
-// launch_conv1d_mfma would run `a` (stride 1) on the chunked small-conv
-// kernel as a 1x1 GEMM: the launches that can take ln_stat
-bool conv1d_mfma_chunked_1x1(const ConvLaunch& a);
 // launch_conv1d_mfma would run `a` as a 1x1 GEMM on split products (one group
-// with weights in two parts, C_in > 256, no input activation)
+// with weights in two parts, C_in > 256, no input activation): the launches
+// that can take ln_stat, stat_out and res_stat
 bool conv1x1_split_ok(const ConvLaunch& a);
 // Scratch floats a launch needs for split-K partial sums (0: no split).
 size_t conv1d_mfma_split_floats(const ConvLaunch& a);

@@ -80,3 +80,12 @@ def test_uneven_shares_of_the_waves(hidden, ffn, L):
     """Widths whose 16-channel steps do not divide evenly among the four or
     eight waves of a tile, with the LayerNorm applied on the way in."""
     assert _other_width(hidden, ffn, L) < 5e-6
+
+
+@pytest.mark.parametrize("hidden,ffn,L", [(192, 768, 40), (288, 3072, 40), (288, 3072, 300), (480, 1920, 70),
+                                          (384, 1500, 40)])
+def test_widths_the_split_products_do_not_take(hidden, ffn, L):
+    """At most 256 channels, or not a multiple of 64: the fp32 GEMMs, among them
+    the 3072-channel reduction in two splits with its reduce launch, and the
+    LayerNorms as launches of their own."""
+    assert _other_width(hidden, ffn, L) < 5e-6
