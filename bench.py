@@ -47,6 +47,8 @@ PEAK_HBM_GBS = 8000.0
 PEAK_BF16_TFLOPS = 2500.0  # dense bf16 MFMA
 # fp32 convolutions on the fp16 matrix cores: three fp16 products per fp32 product
 PEAK_SPLIT_TFLOPS = PEAK_BF16_TFLOPS / 3
+# a fused pair of convolutions counts as two launches, as the session's timing counts it
+RESBLOCK_KERNELS = "resblock_pair + conv1d_split (GeneratorNSF ResBlock convs, all stages)"
 SR = 40000
 P_FRAMES = 1000           # 10 s at 100 frames/s
 CPU_SAMPLE_FRAMES = 400   # 4 s sample for the numpy baseline (about 10 s of CPU work)
@@ -270,7 +272,7 @@ def bench_dec48(args):
     n = max(rb["launches"], 1)
     avg_s = rb["ms"] / 1e3 / n
     achieved = rb["flops"] / n / avg_s / 1e12 if avg_s > 0 else 0.0
-    roofline = {"kernel": "conv1d_split (GeneratorNSF ResBlock convs, all stages)", "bound": "mfma",
+    roofline = {"kernel": RESBLOCK_KERNELS, "bound": "mfma",
                 "achieved": round(achieved, 2), "peak": round(PEAK_SPLIT_TFLOPS, 1), "unit": "TFLOP/s",
                 "frac": round(achieved / PEAK_SPLIT_TFLOPS, 4), "traffic": None,
                 "avg_launch_us": round(avg_s * 1e6, 2), "launches_per_step": n // args.steps,
@@ -366,7 +368,7 @@ def bench_bf16(args, precision):
     n_launch = max(rb["launches"], 1)
     avg_s = rb["ms"] / 1e3 / n_launch
     achieved = rb["flops"] / n_launch / avg_s / 1e12 if avg_s > 0 else 0.0
-    roofline = {"kernel": "conv1d_" + ("bf16" if precision >= 2 else "split") + " (GeneratorNSF ResBlock convs)",
+    roofline = {"kernel": RESBLOCK_KERNELS + (", bf16" if precision >= 2 else ""),
                 "bound": "mfma", "achieved": round(achieved, 2), "peak": peak_rb, "unit": "TFLOP/s",
                 "frac": round(achieved / peak_rb, 4), "traffic": None,
                 "avg_launch_us": round(avg_s * 1e6, 2), "launches_per_step": n_launch // args.steps,
@@ -477,7 +479,7 @@ def bench_vc(args):
     n = max(rb["launches"], 1)
     avg_s = rb["ms"] / 1e3 / n
     achieved = rb["flops"] / n / avg_s / 1e12 if avg_s > 0 else 0.0
-    roofline = {"kernel": "conv1d_split (GeneratorNSF ResBlock convs, all stages)", "bound": "mfma",
+    roofline = {"kernel": RESBLOCK_KERNELS, "bound": "mfma",
                 "achieved": round(achieved, 2), "peak": round(PEAK_SPLIT_TFLOPS, 1), "unit": "TFLOP/s",
                 "frac": round(achieved / PEAK_SPLIT_TFLOPS, 4), "traffic": None,
                 "avg_launch_us": round(avg_s * 1e6, 2), "launches_per_step": n // args.steps,
@@ -674,7 +676,7 @@ def main():
     avg_s = rb["ms"] / 1e3 / n_launch
     flops_launch = rb["flops"] / n_launch
     achieved = flops_launch / avg_s / 1e12 if avg_s > 0 else 0.0
-    roofline = {"kernel": "conv1d_split (GeneratorNSF ResBlock convs, all stages)", "bound": "mfma",
+    roofline = {"kernel": RESBLOCK_KERNELS, "bound": "mfma",
                 "achieved": round(achieved, 2), "peak": round(PEAK_SPLIT_TFLOPS, 1), "unit": "TFLOP/s",
                 "frac": round(achieved / PEAK_SPLIT_TFLOPS, 4), "traffic": profiled_traffic(),
                 "algorithmic_bytes": int(rb["bytes"] / n_launch),
