@@ -11,10 +11,12 @@
 // are 2.7 times as many: whole waveforms against 64 bits, fp32 matrix cores ->
 // here, 1 s at 40k 2.3e-6 -> 1.4e-6, 10 s 1.7e-6 -> 1.4e-6, 48k decoder 1.5e-6
 // -> 1.3e-6.  The instruction does 16 times the multiply-adds per cycle of
-// v_mfma_f32_32x32x2_f32; three products leave a factor of 16 / 3.  What
-// bounds the large launches is power: the clock falls to 1.8 GHz and a loop of
-// nothing but these instructions on random data holds 1700 TFLOP/s, a third
-// of which is 570 of fp32 products.  (Three bf16 parts, six products: the same
+// v_mfma_f32_32x32x2_f32; three products leave a factor of 16 / 3.  Under them
+// the clock falls to 1.63 GHz, where matrix cores that never paused would do
+// 1710 TFLOP/s, 570 of fp32 products (a loop of nothing but these instructions
+// holds 1700).  The 256-channel launches at 10 000 columns keep them busy 0.57
+// of the cycles (SQ counters), the rest being waits for operands and barriers:
+// 320 TFLOP/s.  (Three bf16 parts, six products: the same
 // launches at 190 - 220 TFLOP/s of fp32 products, error 1.6e-6.)
 //
 // Range: weights are scaled per output row to a largest value in [2^9, 2^10),

@@ -4,8 +4,12 @@
 // with K taps, conv1 at dilation d and conv2 at 1.  Up to three groups (the
 // ResBlocks of a stage, K = 3, 7, 11) share a grid, heaviest first.
 //
-// Bound by the matrix cores at the clock their power allows, and at C = 32
-// by HBM: run as two launches the intermediate crosses it twice, and the second
+// Bound by the matrix cores where channels are many: at 128 they are busy 0.67 of
+// the cycles at the 1.63 GHz the clock falls to (SQ counters), at 64 0.54, the
+// rest being waits for operands, barriers and the two epilogues (2.5 and 4.3 VALU
+// instructions an MFMA).  At 32 channels (0.41) HBM bounds it: 538 MB in 140 us,
+// 0.8 of the card's copy rate.  Run as two launches the intermediate crosses HBM
+// twice, and at 32 channels the second
 // launch moved 444 MB in 104 us, the card's copy rate.  Here a workgroup owns
 // all C channels of BN intermediate columns.  It forms them (the staging and
 // main loop of conv1d_split_kernel), applies bias and leaky ReLU in registers,
