@@ -89,3 +89,25 @@ def test_widths_the_split_products_do_not_take(hidden, ffn, L):
     the 3072-channel reduction in two splits with its reduce launch, and the
     LayerNorms as launches of their own."""
     assert _other_width(hidden, ffn, L) < 5e-6
+
+
+def test_a_click_takes_nothing_from_its_neighbours(weights):
+    """Two opposite clicks of 1e6 in noise of 1e-3, no GroupNorm bias: the frames
+    beside them share tiles of the first stride-2 conv with theirs, 2^27 times as
+    large.  What the normalisation leaves of the noise is off by about 1e-3 on
+    either side (its rounding), beside the clicks as elsewhere."""
+    sd = dict(weights)
+    key = "feature_extractor.conv_layers.0.layer_norm.bias"
+    sd[key] = np.zeros_like(sd[key])
+    x = 1e-3 * np.random.default_rng(1).standard_normal((1, 34000), dtype=np.float32)
+    x[0, 16000], x[0, 16400] = 1e6, -1e6
+    with nn_ref.conv_formulation("taps"):
+        want = hubert_ref.HubertRef(sd).feature_extractor(x)[0]  # [106][512]
+    m = HipHubert(sd)
+    m.encode(x)
+    got = m.read("feats", (512, 106)).T
+    m.close()
+    off = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    beside = np.r_[off[44:49], off[52:57]]
+    assert (off[49:52] < 5e-6).all()
+    assert beside.max() < 1.6 * np.median(off)
